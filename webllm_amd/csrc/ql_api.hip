@@ -19,7 +19,10 @@ struct ql_ctx {
     int device;
     hipStream_t stream;
     uint32_t* counters;   // split-K arrival counters; every launch leaves them at zero
-    float* attn_ws;       // attention key-split partials (ql::kAttnWsBytes), used in stream order
+    float* attn_ws;       // ql::kAttnWsBytes, used in stream order: attention key-split partials, the
+                          // many-row fp16 product's image of x
+    std::mutex ws_lock;   // held while the launches that pass data through attn_ws are enqueued, so
+                          // that another thread's do not come between them
     float* noalloc_scratch;  // this device's address of `scratch` (ql_linear_noalloc)
     hipEvent_t ev_start, ev_stop;
     bool capturing;
@@ -1992,7 +1995,8 @@ int ql_gemv_f16w(ql_ctx* ctx, const ql_arena* weights, uint64_t w_off, uint64_t 
     a.M = M;
     a.N = N;
     a.K = K;
-    QL_HIP(ql::launch_gemv_f16w(a, ql::gemv_f16w_fast_ok(M, N, K), ctx->cu_count, ctx->stream));
+    std::lock_guard<std::mutex> guard(ctx->ws_lock);
+    QL_HIP(ql::launch_gemv_f16w(a, ql::gemv_f16w_fast_ok(M, N, K), ctx->cu_count, ctx->attn_ws, ql::kAttnWsBytes, ctx->stream));
     return QL_OK;
 }
 
@@ -2112,6 +2116,7 @@ int ql_attention_decode(ql_ctx* ctx, ql_arena* act, uint64_t q_off, const ql_are
     a.past = past_len;
     a.scale = (float)(1.4426950408889634 / std::sqrt((double)D));   // log2(e) / sqrt(D): scores in base-2 units
     if (ql::plan_attention(&a)) return fail(QL_E_INVALID, "attention shape does not fit the workspace");
+    std::lock_guard<std::mutex> guard(ctx->ws_lock);
     QL_HIP(ql::launch_attention(a, ctx->stream));
     return QL_OK;
 }

@@ -175,7 +175,12 @@ struct F16wArgs {
 };
 bool gemv_f16w_fast_ok(int M, int N, int K);
 size_t gemv_f16w_lds(int M, int K);
-hipError_t launch_gemv_f16w(const F16wArgs& a, bool fast, int cu_count, hipStream_t stream);
+// ws: a workspace for the many-row form's image of x, used in stream order
+hipError_t launch_gemv_f16w(const F16wArgs& a, bool fast, int cu_count, void* ws, size_t ws_bytes, hipStream_t stream);
+// More rows than one pass of the GEMV (ql_f16w_gemm.hip): K % 8 == 0; gemm_f16w_rows gives the rows per
+// image that fit ws_bytes (below 16: K too long).
+int gemm_f16w_rows(int K, size_t ws_bytes);
+hipError_t launch_gemm_f16w(const F16wArgs& a, int cu_count, void* ws, size_t ws_bytes, hipStream_t stream);
 
 // The embedding lookup over the fp16 table: out[r, :] = f32(w[tokens[r], :]).
 struct EmbedArgs {
