@@ -208,12 +208,14 @@ int ql_kv_store(ql_ctx* ctx, const ql_arena* act, uint64_t src_off, ql_arena* ca
  *   reference/qwen-ref.ts:65-111 attentionGqaRef). q and out are [M, n_head, D] fp32 in `act`;
  *   D = 4..256 (multiple of 4); past_len + M <= max_t and <= 8192. fp32 throughout. Few rows x heads
  *   (decode) split the keys over workgroups, with partials in a 4 MiB workspace the context owns:
- *   calls on one context run in its stream's order, so they never share it at the same time. */
+ *   calls on one context run in its stream's order, so they never share it at the same time. Many rows
+ *   (M >= 96 with past_len + M / 2 >= 896, D 64 or 128: prefill) run as tiles of 128 (row, head) pairs on
+ *   the matrix cores, operands as two fp16 parts, with a 64 MiB workspace of the context's. */
 int ql_attention_decode(ql_ctx* ctx, ql_arena* act, uint64_t q_off, const ql_arena* cache, uint64_t k_off,
                         uint64_t v_off, int32_t max_t, int32_t M, int32_t n_head, int32_t n_kv_head, int32_t D,
                         int32_t past_len, uint64_t out_off);
-/* ql_plan_attention (diagnostic, host only): the launch shape ql_attention_decode picks for these
- *   dimensions, with the same checks (no counterpart in the reference, whose attention is one
+/* ql_plan_attention (diagnostic, host only): the launch shape ql_attention_decode's row-per-workgroup
+ *   kernel has for these dimensions, with the same checks (no counterpart in the reference, whose attention is one
  *   dispatch per layer, qwen.ts:430-442). heads_per_run query heads share each K/V row read;
  *   nsplit key splits (1 = no merge launch); workgroups of the attention launch. */
 typedef struct ql_attn_info {

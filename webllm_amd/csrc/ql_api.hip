@@ -21,7 +21,8 @@ struct ql_ctx {
     uint32_t* counters;   // split-K arrival counters; every launch leaves them at zero
     float* attn_ws;       // ql::kAttnWsBytes, used in stream order: attention key-split partials, the
                           // many-row fp16 product's image of x
-    std::mutex ws_lock;   // held while the launches that pass data through attn_ws are enqueued, so
+    void* tile_ws;        // ql::kAttnTileWsBytes, likewise: the many-row attention's images and partials
+    std::mutex ws_lock;   // held while the launches that pass data through them are enqueued, so
                           // that another thread's do not come between them
     float* noalloc_scratch;  // this device's address of `scratch` (ql_linear_noalloc)
     hipEvent_t ev_start, ev_stop;
@@ -1495,6 +1496,7 @@ int ql_create(int device, ql_ctx** out)
     if ((e = hipMalloc(&c->counters, sizeof(uint32_t) * ql::kCounterCapacity)) != hipSuccess ||
         (e = hipMemset(c->counters, 0, sizeof(uint32_t) * ql::kCounterCapacity)) != hipSuccess ||
         (e = hipMalloc(&c->attn_ws, ql::kAttnWsBytes)) != hipSuccess ||
+        (e = hipMalloc(&c->tile_ws, ql::kAttnTileWsBytes)) != hipSuccess ||
         (e = scratch_address(device, &c->noalloc_scratch)) != hipSuccess ||
         (e = hipEventCreate(&c->ev_start)) != hipSuccess ||
         (e = hipEventCreate(&c->ev_stop)) != hipSuccess) {
@@ -1515,6 +1517,7 @@ int ql_destroy(ql_ctx* ctx)
     (void)hipEventDestroy(ctx->ev_stop);
     (void)hipFree(ctx->counters);
     (void)hipFree(ctx->attn_ws);
+    (void)hipFree(ctx->tile_ws);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return QL_OK;
@@ -2117,6 +2120,11 @@ int ql_attention_decode(ql_ctx* ctx, ql_arena* act, uint64_t q_off, const ql_are
     a.scale = (float)(1.4426950408889634 / std::sqrt((double)D));   // log2(e) / sqrt(D): scores in base-2 units
     if (ql::plan_attention(&a)) return fail(QL_E_INVALID, "attention shape does not fit the workspace");
     std::lock_guard<std::mutex> guard(ctx->ws_lock);
+    int tile_split;
+    if (ql::attention_tile_ok(a, ql::kAttnTileWsBytes, &tile_split)) {
+        QL_HIP(ql::launch_attention_tile(a, ctx->tile_ws, tile_split, ctx->stream));
+        return QL_OK;
+    }
     QL_HIP(ql::launch_attention(a, ctx->stream));
     return QL_OK;
 }

@@ -1,0 +1,502 @@
+// Attention of many query rows over the KV cache (prefill: ql_attention_decode with M rows) on the
+// matrix cores: the tiled form of attn_kernel (ql_attn.hip), which gives every query row a workgroup
+// of its own and re-reads that row's keys.
+//
+// fp32 in, fp32 out, fp32-grade throughout: every operand enters as two fp16 parts, x 2^s = hi + lo
+// (about 22 bits), and a product is lo.hi + hi.lo + hi.hi in fp32 on v_mfma_f32_16x16x32_f16, three of
+// which cost 3/16 of the fp32 MFMA's time.
+//
+// 1. attn_image_kernel splits K and V once, per kv head and block of 64 keys, into the fragments the
+//    MFMAs read. K has one exponent per block (a score's error is absolute: 2^-37 of the block's
+//    largest), V one per block and column d. It notes blocks that hold an infinity or NaN.
+// 2. attn_tile_kernel: a workgroup has 128 (query row, head) pairs of one kv head, ordered row-major so
+//    that their causal limits are close; wave w has 32. Scores are computed transposed, S^T = K Q^T
+//    (lane = query column, registers = keys), so that after the exponential a lane already holds the
+//    B fragment of O^T = V^T P^T for the keys {4g .. 4g+3} of each 16; V's image has its keys in that
+//    order and P never leaves its registers. Per block: K from LDS while V's loads are in flight, then
+//    V from LDS while the next K's are, two barriers. Running max and sums in fp32 as in attn_kernel;
+//    P's parts are taken of 2^14 P (fp16's range), after the exponential: 14 added to its argument
+//    would round away the bits that make it exact. A block's P.V starts
+//    from zero and is added to the fp32 output by the VALU, so the matrix unit never carries the long sum.
+// 3. Where the row blocks do not fill the chip the keys are split over workgroups and
+//    attn_merge_kernel adds the splits.
+//
+// What bounds it: per block and wave 192 MFMAs, 64 KB of LDS reads and the softmax's vector work (some
+// 400 instructions), which overlap only as far as the CU's two workgroups are in different phases. 28 / 4
+// heads of 128, 1024 rows after 1024 keys: images 9 us, tiles 95 us (760 TFLOP/s of fp16 products), merge
+// 9 us; attn_kernel took 630 us.
+//
+// A masked key has P = 0, which an infinity or NaN in its V would turn into NaN; rows before that key
+// must not see it. Where the image kernel noted one, the kv head's workgroups walk their rows one by
+// one in fp32 instead (row_by_row).
+#include <algorithm>
+
+#include "ql_device.h"
+#include "ql_digits.h"
+#include "ql_internal.h"
+
+namespace ql {
+
+namespace {
+
+constexpr int kBlk = 64;                 // keys per block
+constexpr int kRows = 128;               // (row, head) pairs per workgroup
+constexpr int kWorkgroups = 512;         // two per CU
+constexpr float kPScale = 16384.f;       // P enters the MFMA times this, V's factors carry its inverse
+
+__device__ __forceinline__ float ex2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// s with |mx| 2^s in [2^14, 2^15); 0 for zero
+__device__ __forceinline__ int shift_of(float mx) { return mx > 0.f && mx <= 3.4028235e38f ? 14 - ilogbf(mx) : 0; }
+
+__device__ __forceinline__ void split8(const float (&x)[8], f16x8& hi, f16x8& lo)
+{
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        hi[e] = (_Float16)x[e];
+        lo[e] = (_Float16)(x[e] - (float)hi[e]);
+    }
+}
+
+struct AttnTile {
+    const float *q, *k, *v;
+    float *out, *ws;                     // ws: key-split partials, as attn_kernel's
+    u32x4 *kimg, *vimg;                  // [KV][blocks][16 D units]
+    float *ksc, *vsc;                    // [KV][blocks] and [KV][blocks][D]: 2^-s
+    uint32_t* bad;                       // [KV][blocks][2]
+    int M, H, KV, G, past, T, blocks, nsplit;
+    float scale;
+};
+
+// blockIdx: (block, kv head, 0: K or 1: V)
+template <int ND>
+__global__ __launch_bounds__(256) void attn_image_kernel(const AttnTile a)
+{
+    constexpr int D = 16 * ND, NK = D / 32, LD = D + 1;
+    __shared__ float tile[kBlk * LD];
+    __shared__ float red[256];
+    const int b = blockIdx.x, kv = blockIdx.y, tid = threadIdx.x;
+    const bool isv = blockIdx.z;
+    const int row_len = a.KV * D;
+    const float* src = (isv ? a.v : a.k) + (size_t)kv * D;
+    float mx = 0.f;
+    bool fin = true;
+    for (int i = tid; i < kBlk * (D / 4); i += 256) {
+        const int r = i / (D / 4), c = i % (D / 4), key = b * kBlk + r;
+        const f32x4 x = key < a.T ? ld_global(reinterpret_cast<const f32x4*>(src + (size_t)key * row_len) + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            tile[r * LD + 4 * c + e] = x[e];
+            mx = fmaxf(mx, fabsf(x[e]));
+            fin = fin && fabsf(x[e]) <= 3.4028235e38f;
+        }
+    }
+    const bool all_fin = __syncthreads_and(fin);
+    const size_t blk = (size_t)kv * a.blocks + b;
+    if (tid == 0) a.bad[2 * blk + isv] = all_fin ? 0u : 1u;
+    if (!isv) {
+        red[tid] = mx;
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if (tid < o) red[tid] = fmaxf(red[tid], red[tid + o]);
+            __syncthreads();
+        }
+        const int sh = shift_of(red[0]);
+        if (tid == 0) a.ksc[blk] = ldexpf(1.f, -sh);
+        // unit (kt, t, part, lane (i, g)): K[16 kt + i][32 t + 8 g .. + 7]
+        u32x4* dst = a.kimg + blk * (16 * D);
+        for (int u = tid; u < 4 * NK * 64; u += 256) {
+            const int lane = u & 63, kt_t = u >> 6, kt = kt_t / NK, t = kt_t % NK;
+            const float* p = tile + (16 * kt + (lane & 15)) * LD + 32 * t + 8 * (lane >> 4);
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = ldexpf(p[e], sh);
+            f16x8 hi, lo;
+            split8(x, hi, lo);
+            st_global(dst + kt_t * 128 + lane, __builtin_bit_cast(u32x4, hi));
+            st_global(dst + kt_t * 128 + 64 + lane, __builtin_bit_cast(u32x4, lo));
+        }
+    } else {
+        // column maxima: 256 / D threads a column, then one
+        constexpr int P = 256 / D;
+        const int d = tid % D, part = tid / D;
+        float cm = 0.f;
+        for (int r = part; r < kBlk; r += P) cm = fmaxf(cm, fabsf(tile[r * LD + d]));
+        red[tid] = cm;
+        __syncthreads();
+        if (tid < D) {
+#pragma unroll
+            for (int o = 1; o < P; o++) cm = fmaxf(cm, red[tid + o * D]);
+            const int sh = shift_of(cm);
+            a.vsc[blk * D + tid] = ldexpf(1.f / kPScale, -sh);
+            red[tid] = (float)sh;
+        }
+        __syncthreads();
+        // unit (dt, ks, part, lane (i, g)): V[32 ks + {4 g + e, 16 + 4 g + e}, e < 4][16 dt + i]
+        u32x4* dst = a.vimg + blk * (16 * D);
+        for (int u = tid; u < ND * 2 * 64; u += 256) {
+            const int lane = u & 63, ks = (u >> 6) & 1, dt = u >> 7;
+            const int c = 16 * dt + (lane & 15), r0 = 32 * ks + 4 * (lane >> 4), sh = (int)red[c];
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = ldexpf(tile[(r0 + (e & 3) + (e >> 2) * 16) * LD + c], sh);
+            f16x8 hi, lo;
+            split8(x, hi, lo);
+            st_global(dst + (u >> 6) * 128 + lane, __builtin_bit_cast(u32x4, hi));
+            st_global(dst + (u >> 6) * 128 + 64 + lane, __builtin_bit_cast(u32x4, lo));
+        }
+    }
+}
+
+// One (row, head) pair after the other, a wave each, D / 64 values a lane, fp32: for kv heads whose
+// cache holds an infinity or NaN (a row must only see its own keys' values).
+template <int ND>
+__device__ __forceinline__ void row_by_row(const AttnTile& a, int kvh, int r0, int r1, int k0, int k1, int split)
+{
+    constexpr int D = 16 * ND, E = D / 64;
+    const int lane = threadIdx.x & 63;
+    for (int r = r0; r < r1; r++) {
+        const int m = r / a.G;
+        const size_t row = (size_t)m * a.H + kvh * a.G + (r - m * a.G);
+        float qv[E], acc[E], mr = -INFINITY, l = 0.f;
+        for (int e = 0; e < E; e++) {
+            qv[e] = a.q[row * D + lane + 64 * e];
+            acc[e] = 0.f;
+        }
+        const int end = min(k1, a.past + m + 1);
+        for (int key = k0; key < end; key++) {
+            const size_t off = ((size_t)key * a.KV + kvh) * D + lane;
+            float dot = 0.f;
+            for (int e = 0; e < E; e++) dot = fmaf(qv[e], a.k[off + 64 * e], dot);
+            for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o);
+            const float s = dot * a.scale, mn = fmaxf(mr, s);
+            if (mn == -INFINITY) continue;               // no visible key so far has a score above -inf
+            const float c = ex2(mr - mn), p = ex2(s - mn);
+            l = l * c + p;
+            for (int e = 0; e < E; e++) acc[e] = fmaf(p, a.v[off + 64 * e], acc[e] * c);
+            mr = mn;
+        }
+        if (a.nsplit == 1) {
+            const float inv = 1.f / l;
+            for (int e = 0; e < E; e++) a.out[row * D + lane + 64 * e] = acc[e] * inv;
+        } else {
+            const size_t slot = row * a.nsplit + split;
+            for (int e = 0; e < E; e++) a.ws[slot * D + lane + 64 * e] = acc[e];
+            float* st = a.ws + (size_t)a.M * a.H * a.nsplit * D + 2 * slot;
+            if (lane < 2) st[lane] = lane ? l : mr;
+        }
+    }
+}
+
+template <int ND>
+__global__ __launch_bounds__(256, 2) void attn_tile_kernel(const AttnTile a)
+{
+    constexpr int D = 16 * ND, NK = D / 32;
+    constexpr int U = 16 * D;                            // 16-byte units of a block's K or V image
+    constexpr int TU = U / 256;
+    __shared__ u32x4 kb[U], vb[U];
+    __shared__ float vscale[D];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15, g = lane >> 4;
+    // the longest causal ranges first
+    const int rb = gridDim.x - 1 - blockIdx.x, split = blockIdx.y, kvh = blockIdx.z;
+    const int R = a.M * a.G;
+    const int kend = a.past + (min(rb * kRows + kRows, R) - 1) / a.G + 1;
+    const int nblk = (kend + kBlk - 1) / kBlk, per = (nblk + a.nsplit - 1) / a.nsplit;
+    const int b0 = min(nblk, split * per), b1 = min(nblk, b0 + per);
+    const int w0 = rb * kRows + wave * 32;               // the wave's first pair
+    const size_t blk0 = (size_t)kvh * a.blocks;
+    uint32_t flag = 0;
+    for (int i = lane; i < 2 * nblk; i += 64) flag |= a.bad[2 * blk0 + i];
+    if (__any(flag != 0)) {                              // the same for every wave of the workgroup
+        row_by_row<ND>(a, kvh, w0, min(w0 + 32, R), b0 * kBlk, min(b1 * kBlk, a.T), split);
+        return;
+    }
+
+    // Q fragments and exponents: lane (i, g) holds row i's values 32 t + 8 g .. + 7
+    f16x8 qh[2][NK], ql[2][NK];
+    float qs[2];
+    int lim[2];                                          // last visible key
+    size_t qrow[2];
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++) {
+        const int r = min(w0 + 16 * mt + i16, R - 1), m = r / a.G;
+        lim[mt] = a.past + m;
+        qrow[mt] = (size_t)m * a.H + kvh * a.G + (r - m * a.G);
+        const f32x4* p = reinterpret_cast<const f32x4*>(a.q + qrow[mt] * D) + 2 * g;
+        f32x4 x[NK][2];
+        float mx = 0.f;
+#pragma unroll
+        for (int t = 0; t < NK; t++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                x[t][h] = ld_global(p + 8 * t + h);
+#pragma unroll
+                for (int e = 0; e < 4; e++) mx = fmaxf(mx, fabsf(x[t][h][e]));
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const int sh = shift_of(mx);
+        qs[mt] = ldexpf(a.scale, -sh);
+#pragma unroll
+        for (int t = 0; t < NK; t++) {
+            float y[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) y[e] = ldexpf(x[t][e >> 2][e & 3], sh);
+            split8(y, qh[mt][t], ql[mt][t]);
+        }
+    }
+    const int free_key = a.past + min(w0, R - 1) / a.G;  // keys up to here are visible to the whole wave
+
+    f32x4 acc[ND][2];
+    float mr[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < ND; d++) acc[d][0] = acc[d][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    u32x4 st[TU];
+    const u32x4* kp = a.kimg + blk0 * U + tid;
+    const u32x4* vp = a.vimg + blk0 * U + tid;
+    auto load = [&](const u32x4* p, int b) {
+#pragma unroll
+        for (int u = 0; u < TU; u++) st[u] = ld_global(p + (size_t)b * U + u * 256);
+    };
+    auto put = [&](u32x4* lds) {
+#pragma unroll
+        for (int u = 0; u < TU; u++) lds[u * 256 + tid] = st[u];
+    };
+    if (b0 < b1) {
+        load(kp, b0);
+        put(kb);
+    }
+    for (int b = b0; b < b1; b++) {
+        __syncthreads();                                 // K of block b is in LDS; V's buffer is free
+        load(vp, b);
+        const float vs1 = ld_global(a.vsc + (blk0 + b) * D + (tid & (D - 1)));
+        const float ks = ld_global(a.ksc + blk0 + b);
+        f32x4 s[4][2];
+#pragma unroll
+        for (int kt = 0; kt < 4; kt++) {
+            s[kt][0] = s[kt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            // the small products first: the sum takes its full size, and the roundings that go with it,
+            // only in the last NK
+            f16x8 kh[NK];
+#pragma unroll
+            for (int t = 0; t < NK; t++) {
+                const u32x4* p = kb + (kt * NK + t) * 128 + lane;
+                kh[t] = __builtin_bit_cast(f16x8, p[0]);
+                const f16x8 kl = __builtin_bit_cast(f16x8, p[64]);
+#pragma unroll
+                for (int mt = 0; mt < 2; mt++) s[kt][mt] = mfma_16x16x32_f16(kl, qh[mt][t], s[kt][mt]);
+#pragma unroll
+                for (int mt = 0; mt < 2; mt++) s[kt][mt] = mfma_16x16x32_f16(kh[t], ql[mt][t], s[kt][mt]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < NK / 2; t++) s[kt][mt] = mfma_16x16x32_f16(kh[t], qh[mt][t], s[kt][mt]);
+#pragma unroll
+                for (int t = NK / 2; t < NK; t++) z = mfma_16x16x32_f16(kh[t], qh[mt][t], z);
+                s[kt][mt] += z;
+            }
+        }
+        if (b * kBlk + kBlk - 1 > free_key)
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+#pragma unroll
+                    for (int mt = 0; mt < 2; mt++)
+                        if (b * kBlk + 16 * kt + 4 * g + r > lim[mt]) s[kt][mt][r] = -INFINITY;
+        f16x8 ph[2][2], pl[2][2];                        // [step of 32 keys][row tile]
+        float al[2];
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) {
+            const float f = fmaxf(qs[mt] * ks, 1.17549435e-38f);
+            float bm = s[0][mt][0];
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) bm = fmaxf(bm, s[kt][mt][r]);
+            bm = fmaxf(bm, __shfl_xor(bm, 16));
+            bm = fmaxf(bm, __shfl_xor(bm, 32));
+            const float mn = fmaxf(mr[mt], bm * f);
+            const float ref = mn == -INFINITY ? 0.f : mn;         // no visible key yet: every P is 0
+            al[mt] = ex2(mr[mt] - ref);
+            mr[mt] = mn;
+            float sum = 0.f;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                float p[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    p[e] = ex2(fmaf(s[2 * h + (e >> 2)][mt][e & 3], f, -ref));
+                    sum += p[e];
+                    p[e] *= kPScale;
+                }
+                split8(p, ph[h][mt], pl[h][mt]);
+            }
+            l[mt] = l[mt] * al[mt] + sum;
+        }
+        if (__any(al[0] != 1.f || al[1] != 1.f))
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+#pragma unroll
+                for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[d][mt][r] *= al[mt];
+        put(vb);
+        if (tid < D) vscale[tid] = vs1;
+        __syncthreads();                                 // V of block b is in LDS; K's buffer is free
+        load(kp, min(b + 1, b1 - 1));
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            const u32x4* p = vb + d * 256 + lane;
+            const f16x8 vh0 = __builtin_bit_cast(f16x8, p[0]), vl0 = __builtin_bit_cast(f16x8, p[64]);
+            const f16x8 vh1 = __builtin_bit_cast(f16x8, p[128]), vl1 = __builtin_bit_cast(f16x8, p[192]);
+            const f32x4 sc = *reinterpret_cast<const f32x4*>(vscale + 16 * d + 4 * g);
+            f32x4 o[2];
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) o[mt] = mfma_16x16x32_f16(vl0, ph[0][mt], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) o[mt] = mfma_16x16x32_f16(vl1, ph[1][mt], o[mt]);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) o[mt] = mfma_16x16x32_f16(vh0, pl[0][mt], o[mt]);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) o[mt] = mfma_16x16x32_f16(vh1, pl[1][mt], o[mt]);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) o[mt] = mfma_16x16x32_f16(vh0, ph[0][mt], o[mt]);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) o[mt] = mfma_16x16x32_f16(vh1, ph[1][mt], o[mt]);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[d][mt][r] = fmaf(o[mt][r], sc[r], acc[d][mt][r]);
+        }
+        put(kb);
+    }
+
+    // lane (i, g): pair i of each row tile, values 16 d + 4 g .. + 3
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++) {
+        l[mt] += __shfl_xor(l[mt], 16);
+        l[mt] += __shfl_xor(l[mt], 32);
+        if (w0 + 16 * mt + i16 >= R) continue;
+        if (a.nsplit == 1) {
+            const float inv = 1.f / l[mt];
+            f32x4* o = reinterpret_cast<f32x4*>(a.out + qrow[mt] * D) + g;
+#pragma unroll
+            for (int d = 0; d < ND; d++) st_global(o + 4 * d, f32x4{acc[d][mt][0] * inv, acc[d][mt][1] * inv, acc[d][mt][2] * inv, acc[d][mt][3] * inv});
+        } else {
+            const size_t slot = qrow[mt] * a.nsplit + split;
+            f32x4* o = reinterpret_cast<f32x4*>(a.ws + slot * D) + g;
+#pragma unroll
+            for (int d = 0; d < ND; d++) st_global(o + 4 * d, acc[d][mt]);
+            float* stt = a.ws + (size_t)a.M * a.H * a.nsplit * D + 2 * slot;
+            if (g < 2) st_global(stt + g, g ? l[mt] : mr[mt]);
+        }
+    }
+}
+
+// out = sum_i acc_i 2^(m_i - m) / sum_i l_i 2^(m_i - m) over the splits i in order, four values a thread
+__global__ __launch_bounds__(256) void attn_merge_kernel(const float* ws, float* out, int rows, int D, int S)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x, nc = D / 4;
+    if (i >= rows * nc) return;
+    const int row = i / nc, c = i - row * nc;
+    const f32x2* st = reinterpret_cast<const f32x2*>(ws + (size_t)rows * S * D) + (size_t)row * S;
+    const f32x4* src = reinterpret_cast<const f32x4*>(ws + (size_t)row * S * D) + c;
+    float m = -INFINITY, l = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < S; k++) m = fmaxf(m, ld_global(st + k).x);
+#pragma unroll 4
+    for (int k = 0; k < S; k++) {
+        const f32x2 ml = ld_global(st + k);
+        const f32x4 v = ld_global(src + (size_t)k * nc);
+        const float w = ml.x == -INFINITY ? 0.f : ex2(ml.x - m);
+        l = fmaf(ml.y, w, l);
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = fmaf(v[e], w, o[e]);
+    }
+    const float inv = 1.f / l;
+    st_global(reinterpret_cast<f32x4*>(out + (size_t)row * D) + c, f32x4{o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv});
+}
+
+// bytes of the images, exponents and flags, 256-byte aligned pieces
+size_t image_bytes(int KV, int D, int blocks)
+{
+    const size_t n = (size_t)KV * blocks;
+    return 2 * n * kBlk * D * 4 + ((n * D * 4 + 255) & ~(size_t)255) + ((n * 4 + 255) & ~(size_t)255) + ((n * 8 + 255) & ~(size_t)255);
+}
+
+}  // namespace
+
+// The line between this form and attn_kernel is where both its time and its error against 64 bits are the
+// smaller ones: at least 96 rows that see about 900 keys each on average. Measured (28 / 4 heads of 128; us
+// and relative error, attn_kernel -> this): 1024 rows after 1024 keys 630 -> 109, 2.5e-7 -> 2.1e-7; 128
+// after 1500 93 -> 38, 2.6e-7 -> 2.2e-7; 1024 after 400 416 -> 83, 2.2e-7 -> 2.0e-7. Beyond the line it is
+// mostly still faster but less exact, because attn_kernel's chains of fp32 sums are short there: 1024 rows
+// after none 247 -> 65 us but 1.4e-7 -> 1.5e-7; 48 after 2000 (which attn_kernel splits) 29 -> 20 us but
+// 1.9e-7 -> 2.1e-7 (14 / 2 heads of 64).
+bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit)
+{
+    if (a.D != 64 && a.D != 128) return false;
+    if (a.M < 96 || a.past + a.M / 2 < 896) return false;
+    const int blocks = (a.past + a.M + kBlk - 1) / kBlk;
+    const size_t img = image_bytes(a.KV, a.D, blocks);
+    if (img > ws_bytes) return false;                    // so many kv heads: the general kernel
+    // key splits up to two workgroups a CU (1 split or 4 instead of 2 at 1024 rows: 144, 138 against 131 us
+    // in an earlier form), of at least two blocks, as many as the workspace holds
+    const int rb = (a.M * a.G + kRows - 1) / kRows * a.KV;
+    int s = std::max(1, std::min(kWorkgroups / rb, (blocks + 1) / 2));
+    const size_t one = (size_t)a.M * a.H * (a.D + 2) * sizeof(float);
+    *nsplit = (int)std::min<size_t>(std::min(s, 128), std::max<size_t>(1, (ws_bytes - img) / one));
+    return true;
+}
+
+hipError_t launch_attention_tile(const AttnArgs& a, void* ws, int nsplit, hipStream_t stream)
+{
+    AttnTile t;
+    t.q = a.q;
+    t.k = a.k;
+    t.v = a.v;
+    t.out = a.out;
+    t.M = a.M;
+    t.H = a.H;
+    t.KV = a.KV;
+    t.G = a.G;
+    t.past = a.past;
+    t.T = a.past + a.M;
+    t.blocks = (t.T + kBlk - 1) / kBlk;
+    t.nsplit = nsplit;
+    t.scale = a.scale;
+    const size_t n = (size_t)a.KV * t.blocks;
+    char* p = static_cast<char*>(ws);
+    t.kimg = reinterpret_cast<u32x4*>(p);
+    p += n * kBlk * a.D * 4;
+    t.vimg = reinterpret_cast<u32x4*>(p);
+    p += n * kBlk * a.D * 4;
+    t.vsc = reinterpret_cast<float*>(p);
+    p += (n * a.D * 4 + 255) & ~(size_t)255;
+    t.ksc = reinterpret_cast<float*>(p);
+    p += (n * 4 + 255) & ~(size_t)255;
+    t.bad = reinterpret_cast<uint32_t*>(p);
+    p += (n * 8 + 255) & ~(size_t)255;
+    t.ws = reinterpret_cast<float*>(p);
+    const dim3 ig(t.blocks, a.KV, 2), tg((a.M * a.G + kRows - 1) / kRows, nsplit, a.KV);
+    if (a.D == 64) {
+        hipLaunchKernelGGL(attn_image_kernel<4>, ig, dim3(256), 0, stream, t);
+        hipLaunchKernelGGL(attn_tile_kernel<4>, tg, dim3(256), 0, stream, t);
+    } else {
+        hipLaunchKernelGGL(attn_image_kernel<8>, ig, dim3(256), 0, stream, t);
+        hipLaunchKernelGGL(attn_tile_kernel<8>, tg, dim3(256), 0, stream, t);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || nsplit == 1) return e;
+    const int rows = a.M * a.H;
+    hipLaunchKernelGGL(attn_merge_kernel, dim3((rows * (a.D / 4) + 255) / 256), dim3(256), 0, stream, t.ws, a.out, rows, a.D, nsplit);
+    return hipGetLastError();
+}
+
+}  // namespace ql

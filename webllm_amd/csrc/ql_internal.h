@@ -223,6 +223,11 @@ struct ElemArgs {
 };
 hipError_t launch_add_rmsnorm(const ElemArgs& a, hipStream_t stream);
 hipError_t launch_silu_mul(const float* gate, const float* up, float* y, long long n, hipStream_t stream);
+// Many rows (ql_attn_tile.hip): whether this call takes the tiled form within ws_bytes of workspace,
+// and its key splits
+constexpr size_t kAttnTileWsBytes = 64u << 20;
+bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit);
+hipError_t launch_attention_tile(const AttnArgs& a, void* ws, int nsplit, hipStream_t stream);
 hipError_t launch_attention(const AttnArgs& a, hipStream_t stream);
 hipError_t launch_kv_store(const float* src, float* dst, int rows, int row_len, int pos0, hipStream_t stream);
 
