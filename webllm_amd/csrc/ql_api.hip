@@ -1857,6 +1857,73 @@ bool prefill_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_a
 
 }  // namespace
 
+namespace {
+
+// Decode linears (M <= 16, checked and aligned) over images of x in the context's workspace: one image
+// per distinct x, then one launch. Returns false when it does not apply.
+bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
+                     const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, int* rc)
+{
+    // Where it is the faster one: at M >= 5 everywhere (M = 8, us, gemv_mfma_kernel -> this: K = N = 896
+    // 11.4 -> 8.0, 3584 x 3584 16.6 -> 7.9, 18944 -> 3584 28.8 -> 17.6, 3584 -> 2 x 18944 26.2 -> 22.2; M = 16
+    // 18.4 -> 8.0, 27.6 -> 9.2, 52.8 -> 26.2, 49.4 -> 26.1), at M = 3, 4 for narrow linears with a long K, whose
+    // K split there costs round trips (M = 4: 3584 x 3584 11.7 -> 8.2, 3584 -> 2 x 18944 20.1 -> 20.7). At
+    // M = 1, 2 the image's launch costs more than it saves.
+    long n = 0;
+    int min_k = INT32_MAX;
+    for (int i = 0; i < count; i++) {
+        n += descs[i].N;
+        min_k = std::min(min_k, descs[i].K);
+    }
+    if (M < 3 || (M < 5 && (n >= 32L * ctx->cu_count || min_k < 2048))) return false;
+    uint64_t off[ql::kMaxBatch], bytes = 0;
+    int first[ql::kMaxBatch];                               // the linear whose image linear i reads
+    for (int i = 0; i < count; i++) {
+        if (!ql::gemv_wave_ok(M, descs[i].N, descs[i].K, descs[i].group)) return false;
+        first[i] = i;
+        for (int k = i - 1; k >= 0; k--)
+            if (x_offs[k] == x_offs[i] && descs[k].K == descs[i].K) first[i] = k;
+        off[i] = first[i] < i ? off[first[i]] : bytes;
+        if (first[i] == i) bytes += align256(ql::x_image_bytes(M, descs[i].K));
+    }
+    if (bytes > ql::kAttnTileWsBytes) return false;
+    if ((*rc = set_device(ctx))) return true;
+    char* ws = static_cast<char*>(ctx->tile_ws);
+    ql::GwBatch b{};
+    ql::XImage im[ql::kMaxBatch];
+    b.count = count;
+    b.M = M;
+    for (int i = 0; i < count; i++) {
+        const ql::GemvLinear g = make_linear(&descs[i], weights);
+        im[i] = ql::XImage{};
+        im[i].x = act->base + x_offs[i];
+        im[i].M = M;
+        im[i].K = descs[i].K;
+        im[i].f16 = x_dtype == QL_DTYPE_F16;
+        ql::x_image_at(&im[i], ws + off[i]);
+        ql::GwLinear& L = b.L[i];
+        L.qweight = g.qweight;
+        L.qzeros = g.qzeros;
+        L.scales = g.scales;
+        L.bias = g.bias;
+        L.img = im[i].img;
+        L.fac = im[i].fac;
+        L.y = reinterpret_cast<float*>(act->base + y_offs[i]);
+        L.N = descs[i].N;
+        L.K = descs[i].K;
+    }
+    ql::gemv_wave_plan(&b, ctx->cu_count);
+    std::lock_guard<std::mutex> guard(ctx->ws_lock);
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < count && e == hipSuccess; i++)
+        if (first[i] == i) e = ql::launch_x_image(im[i], ctx->stream);
+    if (e == hipSuccess) e = ql::launch_gemv_wave(b, ctx->stream);
+    *rc = e == hipSuccess ? QL_OK : hip_fail(e, "launch_gemv_wave");
+    return true;
+}
+
+}  // namespace
+
 int ql_plan_linear(int32_t M, int32_t N, int32_t K, int32_t group, ql_plan* out)
 {
     if (!out) return fail(QL_E_INVALID, "null plan pointer");
@@ -1878,6 +1945,7 @@ int linear_impl(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_
     L.y = reinterpret_cast<float*>(act->base + y_off);
 
     if (p.kind == QL_KIND_GEMV_MFMA && gemv_aligned(d, x_off, y_off)) {
+        if (gemv_wave_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, &rc)) return rc;
         const ql::GemvShape s = ql::gemv_shape(M, d->N, d->K, d->group);
         ql::GemvBatch b{};
         L.split = s.split;
@@ -2273,6 +2341,7 @@ int ql_linear_batch(ql_ctx* ctx, int32_t count, const ql_gptq_desc* descs,
         }
         return QL_OK;
     }
+    if (gemv_wave_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, &rc)) return rc;
     if ((rc = set_device(ctx))) return rc;
     ql::GemvBatch b{};
     b.count = count;

@@ -46,6 +46,38 @@ uint64_t gemv_partial_bytes(int M, int N, int split);
 hipError_t launch_gemv_batch(const GemvBatch& b, hipStream_t stream);
 hipError_t launch_gemv_simple(const GemvLinear& L, int M, int x_dtype, hipStream_t stream);
 
+// Decode product over an image of x (ql_gemv_wave.hip): M <= 16, groups of 128.
+struct XImage {
+    const void* x;             // [M, K] fp32, or fp16 (f16)
+    const float* x2;           // kind 2: [M, K]
+    const float* w;            // kind 1: [K]
+    uint32_t __attribute__((ext_vector_type(4)))* img;
+    float* fac;                // x_image_at sets both in x_image_bytes(M, K) bytes
+    int M, K, kind, f16;       // kind 0: x; 1: rmsnorm(x) * w; 2: silu(x) * x2
+    float eps;
+};
+uint64_t x_image_bytes(int M, int K);
+void x_image_at(XImage* a, void* p);
+hipError_t launch_x_image(const XImage& a, hipStream_t stream);
+struct GwLinear {
+    const uint32_t* qweight;
+    const uint32_t* qzeros;
+    const uint16_t* scales;
+    const float* bias;
+    const float* res;          // [M, N] or nullptr
+    const uint32_t __attribute__((ext_vector_type(4)))* img;
+    const float* fac;
+    float* y;
+    int N, K, wg_begin, pad;
+};
+struct GwBatch {
+    GwLinear L[kMaxBatch];
+    int count, M, nt, wg_total;
+};
+bool gemv_wave_ok(int M, int N, int K, int group);
+void gemv_wave_plan(GwBatch* b, int cu_count);
+hipError_t launch_gemv_wave(const GwBatch& b, hipStream_t stream);
+
 // GEMM (M > 16): y = f16(x) * f16(W)^T, fp32 accumulate.
 struct GemmArgs {
     const uint32_t* qweight;
