@@ -304,7 +304,10 @@ typedef struct ql_seq_info {
     int32_t variant;      /* strips: 1 when the launch is the no-padding kernel on streamed
                              weights (every linear: group 128, K a multiple of 512, N a multiple
                              of 512; M = 5..16, or 2..16 pass by pass); QL_SEQ_PREFILL_PASSES: the
-                             passes that run the chunked split-K GEMM; 0 otherwise */
+                             passes that run the chunked split-K GEMM. ql_seq_get_info, QL_SEQ_TILES: 2
+                             when the created sequence runs its passes as products over activation
+                             images (below; the other figures are then the tiles' plan, launches and
+                             device_bytes its own). 0 otherwise */
     int32_t launches;     /* kernel launches one ql_seq_run enqueues */
 } ql_seq_info;
 /* plan only (host, pure) for a given grid size: validation and the figures above */
@@ -339,6 +342,11 @@ int ql_seq_status(ql_ctx* ctx, ql_seq* seq);
  * fixed order, times the row's 1/rms for an RMSNorm'd input, with bias and residual (and the row
  * sums of squares of outputs a later linear RMSNorms); an external input that is RMSNorm'd adds
  * one launch before its pass. Stream order replaces the device-side waits (nothing can abort).
+ * Other chained sequences (fused or not) with fp32 x, groups of 128, K % 128 == 0 and 16-byte aligned
+ * norm weights run pass by pass over activation images at M = 5..16, and at M = 2..4 where a pass reads
+ * 16 MiB of weights or more on average: per pass, one launch for each distinct input (an RMSNorm, a
+ * SiLU-mul, or rows as they are, as scaled fp16 parts) and one for the pass's linears. ql_plan_seq(_fused)
+ * reports the tiles' plan for them, ql_seq_get_info variant 2 and the launches enqueued.
  * QL_SEQ_PASSES=0 in the environment keeps the tiles. */
 typedef struct ql_seq_fuse {
     uint64_t norm_w_off;

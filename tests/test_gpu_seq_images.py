@@ -1,0 +1,51 @@
+"""GPU: chained decode sequences that run their passes as products over activation images (ql_seq_get_info variant 2:
+M = 5..16, or 2..4 with 16 MiB of weights a pass), every linear against the oracle on the GPU's own inputs, as the tiles'
+tests check them; repeats and graph replays give the same bits."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_fused import FusedModel, _sample, check_fused
+from webllm_amd import qlinear as ql
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = ql.Context(0)
+    yield c
+    c.destroy()
+
+
+@pytest.mark.parametrize("M,layers,C,I,KV", [
+    (5, 2, 256, 640, 128),        # the fewest rows; two layers: residuals and norms of produced rows
+    (8, 1, 896, 4864, 128),       # one fragment, full
+    (9, 1, 384, 128, 128),        # two fragments, one group of K in the down linear
+    (16, 1, 4224, 256, 128),      # RMSNorm rows longer than a workgroup keeps in registers
+    (2, 1, 3584, 18944, 512),     # few rows, large passes
+])
+def test_image_passes_match_oracle(ctx, M, layers, C, I, KV):
+    from oracle import oracle as orc
+    m = FusedModel(ql, ctx, M, layers, C, I, KV)
+    info = m.seq.info
+    assert info.kernel == ql.SEQ_TILES and info.variant == 2 and info.passes == 4 * layers
+    assert info.launches == 8 * layers          # an image and a product per pass: norm, q, norm, SiLU-mul
+    m.seq.run()
+    m.seq.status()
+    first = m.outputs()
+    check_fused(orc, m, first, f"M={M} C={C} I={I}", **({"cols_for": _sample} if C == 3584 else {}))
+    ctx.graph_begin()
+    m.seq.run()
+    g = ctx.graph_end()
+    for _ in range(3):
+        g.launch()
+        m.seq.run()
+        ctx.sync()
+        assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(first, m.outputs()))
+    g.destroy()
+
+
+@pytest.mark.parametrize("M,C,I,variant", [(1, 896, 4864, 0), (4, 896, 4864, 0), (5, 896, 4864, 2)])
+def test_small_passes_of_few_rows_keep_the_tiles(ctx, M, C, I, variant):
+    m = FusedModel(ql, ctx, M, 1, C, I, 128)
+    assert m.seq.info.variant == variant

@@ -46,9 +46,12 @@ struct ql_graph {
 
 // One launch of a pass-by-pass sequence: an RMSNorm into a buffer (e), a SiLU-mul into a buffer
 // (o = silu(g) * u over n values), a pass's strips (s, lds), a pass's part sums (sums), or a
-// pass's prefill GEMM (p) or chunked GEMM (gb).
+// pass's prefill GEMM (p) or chunked GEMM (gb); or an activation image (xi) and a pass's products over
+// images (gw).
 struct SeqStep {
-    enum Kind { kNorm, kGlu, kStrips, kPartSums, kPrefill, kGemm } kind;
+    enum Kind { kNorm, kGlu, kStrips, kPartSums, kPrefill, kGemm, kXImage, kGemvWave } kind;
+    ql::XImage xi{};
+    ql::GwBatch gw{};
     const ql::PartSum* sums = nullptr;   // kPartSums: the device table, count entries
     int count = 0, M = 0, max_n = 0;
     bool glu = false;                    // kPartSums: SiLU-mul entries (part_sum_glu_kernel)
@@ -245,6 +248,23 @@ ql::GemvLinear make_linear(const ql_gptq_desc* d, const ql_arena* w)
     L.K = d->K;
     L.group = d->group;
     L.split = 1;
+    return L;
+}
+
+ql::GwLinear gw_linear(const ql_gptq_desc* d, const ql_arena* w, const ql::XImage& im, float* y, const float* res)
+{
+    const ql::GemvLinear g = make_linear(d, w);
+    ql::GwLinear L{};
+    L.qweight = g.qweight;
+    L.qzeros = g.qzeros;
+    L.scales = g.scales;
+    L.bias = g.bias;
+    L.res = res;
+    L.img = im.img;
+    L.fac = im.fac;
+    L.y = y;
+    L.N = d->N;
+    L.K = d->K;
     return L;
 }
 
@@ -1124,8 +1144,8 @@ bool seq_chained(const std::vector<ql::SeqSpec>& specs)
     return false;
 }
 
-void plan_prefill_passes(const std::vector<ql::SeqSpec>& specs, const ql_seq_fuse* fuse, const uint64_t* x_offs,
-                         int M, int grid, PrefillPasses* P)
+// The passes, their linears and their distinct RMSNorm and SiLU-mul inputs.
+void plan_pass_inputs(const std::vector<ql::SeqSpec>& specs, const ql_seq_fuse* fuse, const uint64_t* x_offs, int M, PrefillPasses* P)
 {
     const int n = (int)specs.size();
     P->depth = seq_pass_of(specs, &P->pass);
@@ -1159,6 +1179,13 @@ void plan_prefill_passes(const std::vector<ql::SeqSpec>& specs, const ql_seq_fus
     }
     P->members.assign(P->depth, {});
     for (int i = 0; i < n; i++) P->members[P->pass[i]].push_back(i);
+}
+
+void plan_prefill_passes(const std::vector<ql::SeqSpec>& specs, const ql_seq_fuse* fuse, const uint64_t* x_offs,
+                         int M, int grid, PrefillPasses* P)
+{
+    const int n = (int)specs.size();
+    plan_pass_inputs(specs, fuse, x_offs, M, P);
     P->plans.assign(P->depth, ql::PrefillPlan{});
     P->chunked.assign(P->depth, 0);
     P->chunk_tiles.assign(P->depth, 0);
@@ -1259,6 +1286,119 @@ uint64_t prefill_passes_bytes(const PrefillPasses& P)
     for (int p = 0; p < P.depth; p++)
         if (!P.chunked[p]) bytes += prefill_layout((int)P.members[p].size(), P.plans[p]).total;
     return bytes;
+}
+
+// ---- chained decode sequences over activation images (M <= 16)
+
+// Where they beat the dependency-ordered tiles, whose tiles each form their activations' digits again:
+// at M >= 5 everywhere, at M = 2..4 where a pass reads so much that its two launches' latency counts
+// little. Measured (us, tiles -> images): 24 layers of the small model (1.9 MB a pass) M = 4 777 -> 842,
+// M = 5 1080 -> 844, M = 8 1273 -> 845, M = 16 2561 -> 963; a layer of the large one (30 MB a pass) M = 2 79 -> 58,
+// M = 5 144 -> 59; between attentions (4 passes and one launch of its own) M = 1 88 -> 90, M = 2 95 -> 76,
+// M = 4 126 -> 77. Sequences that stream their weights from HBM keep the K-part strips (four layers of the
+// large model, M = 8 277 against 311).
+bool image_passes_ok(const std::vector<ql::SeqSpec>& specs, const ql_seq_fuse* fuse, int M, int32_t x_dtype)
+{
+    const char* env = getenv("QL_SEQ_PASSES");
+    if (env && atoi(env) == 0) return false;
+    if (M < 2 || M > ql::kGemvMaxM || x_dtype != QL_DTYPE_F32 || !seq_chained(specs) || passes_ok(specs, M, x_dtype)) return false;
+    uint64_t bytes = 0;
+    for (size_t i = 0; i < specs.size(); i++) {
+        if (!ql::gemv_wave_ok(M, specs[i].N, specs[i].K, specs[i].group)) return false;
+        if ((specs[i].fuse & ql::kFuseNorm) && fuse[i].norm_w_off % 16) return false;
+        bytes += specs[i].weight_bytes;
+    }
+    std::vector<int> pass;
+    return M >= 5 || bytes / std::max(1, seq_pass_of(specs, &pass)) >= (16u << 20);
+}
+
+// Per pass, an image of each distinct input (an RMSNorm, a SiLU-mul, or rows as they are), then the
+// pass's products (launches of up to kMaxBatch linears), bias and residual at the store. The launches run
+// in stream order; nothing waits on the device.
+int image_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
+                        const uint64_t* x_offs, int32_t M, const uint64_t* y_offs, const ql_seq_fuse* fuse,
+                        const std::vector<ql::SeqSpec>& specs, const ql_seq_info& info, ql_seq** out)
+{
+    PrefillPasses P;
+    plan_pass_inputs(specs, fuse, x_offs, M, &P);
+    auto y_ptr = [&](int j) { return reinterpret_cast<float*>(act->base + y_offs[j]); };
+    auto ext_ptr = [&](int src, uint64_t off) -> const float* {
+        return src >= 0 ? y_ptr(src) : reinterpret_cast<const float*>(act->base + off);
+    };
+    // the images: the fused inputs, then one per distinct (rows, width) read as they are
+    std::vector<ql::XImage> image;
+    for (const PrefillPasses::Input& in : P.inputs) {
+        ql::XImage im{};
+        im.x = ext_ptr(in.x_src, in.x_off);
+        im.K = in.K;
+        im.kind = in.glu ? 2 : 1;
+        if (in.glu) im.x2 = ext_ptr(in.x2_src, in.x2_off);
+        else im.w = reinterpret_cast<const float*>(weights->base + in.w_off);
+        im.eps = in.eps;
+        image.push_back(im);
+    }
+    std::vector<int> image_of(n);
+    for (int i = 0; i < n; i++) {
+        image_of[i] = P.input_of[i];
+        if (image_of[i] >= 0) continue;
+        const void* x = ext_ptr(specs[i].src, x_offs[i]);
+        for (size_t k = P.inputs.size(); k < image.size() && image_of[i] < 0; k++)
+            if (image[k].x == x && image[k].K == specs[i].K) image_of[i] = (int)k;
+        if (image_of[i] >= 0) continue;
+        ql::XImage im{};
+        im.x = x;
+        im.K = specs[i].K;
+        image_of[i] = (int)image.size();
+        image.push_back(im);
+    }
+    uint64_t bytes = 0;
+    std::vector<uint64_t> off;
+    for (ql::XImage& im : image) {
+        im.M = M;
+        off.push_back(bytes);
+        bytes += align256(ql::x_image_bytes(M, im.K));
+    }
+    ql_seq* q = new ql_seq();
+    q->device = ctx->device;
+    q->passes = true;
+    const hipError_t e = hipMalloc(&q->dev, bytes);
+    if (e != hipSuccess) {
+        delete q;
+        return hip_fail(e, "ql_seq_create images");
+    }
+    for (size_t k = 0; k < image.size(); k++) ql::x_image_at(&image[k], q->dev + off[k]);
+    std::vector<bool> made(image.size(), false);
+    for (int p = 0; p < P.depth; p++) {
+        const std::vector<int>& mem = P.members[p];
+        for (int i : mem) {
+            if (made[image_of[i]]) continue;
+            made[image_of[i]] = true;
+            SeqStep st{};
+            st.kind = SeqStep::kXImage;
+            st.xi = image[image_of[i]];
+            q->steps.push_back(st);
+        }
+        for (size_t at = 0; at < mem.size(); at += ql::kMaxBatch) {
+            SeqStep st{};
+            st.kind = SeqStep::kGemvWave;
+            ql::GwBatch& b = st.gw;
+            b.M = M;
+            b.count = (int)std::min<size_t>(ql::kMaxBatch, mem.size() - at);
+            for (int k = 0; k < b.count; k++) {
+                const int i = mem[at + k];
+                b.L[k] = gw_linear(&descs[i], weights, image[image_of[i]], y_ptr(i),
+                                   specs[i].fuse & ql::kFuseRes ? ext_ptr(specs[i].res_src, fuse[i].res_off) : nullptr);
+            }
+            ql::gemv_wave_plan(&b, ctx->cu_count);
+            q->steps.push_back(st);
+        }
+    }
+    q->info = info;
+    q->info.device_bytes = bytes;
+    q->info.variant = 2;
+    q->info.launches = (int32_t)q->steps.size();
+    *out = q;
+    return QL_OK;
 }
 
 int prefill_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, const ql_arena* weights,
@@ -1894,23 +2034,13 @@ bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql
     b.count = count;
     b.M = M;
     for (int i = 0; i < count; i++) {
-        const ql::GemvLinear g = make_linear(&descs[i], weights);
         im[i] = ql::XImage{};
         im[i].x = act->base + x_offs[i];
         im[i].M = M;
         im[i].K = descs[i].K;
         im[i].f16 = x_dtype == QL_DTYPE_F16;
         ql::x_image_at(&im[i], ws + off[i]);
-        ql::GwLinear& L = b.L[i];
-        L.qweight = g.qweight;
-        L.qzeros = g.qzeros;
-        L.scales = g.scales;
-        L.bias = g.bias;
-        L.img = im[i].img;
-        L.fac = im[i].fac;
-        L.y = reinterpret_cast<float*>(act->base + y_offs[i]);
-        L.N = descs[i].N;
-        L.K = descs[i].K;
+        b.L[i] = gw_linear(&descs[i], weights, im[i], reinterpret_cast<float*>(act->base + y_offs[i]), nullptr);
     }
     ql::gemv_wave_plan(&b, ctx->cu_count);
     std::lock_guard<std::mutex> guard(ctx->ws_lock);
@@ -2453,6 +2583,11 @@ int seq_create_impl(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, const ql_
     if (M > ql::kGemvMaxM) return prefill_create(ctx, n, descs, weights, act, x_offs, x_dtype, M, y_offs, specs, out);
     if (!fused && ql::strip_eligible(specs, M))
         return strip_create(ctx, n, descs, weights, act, x_offs, x_dtype, M, y_offs, specs, out);
+    if (image_passes_ok(specs, fuse, M, x_dtype)) {
+        ql_seq_info info;
+        if ((rc = plan_seq_impl(n, descs, M, x_offs, x_dtype, y_offs, fuse, ctx->cu_count, &info))) return rc;
+        return image_passes_create(ctx, n, descs, weights, act, x_offs, M, y_offs, fuse, specs, info, out);
+    }
     if (passes_ok(specs, M, x_dtype))
         return passes_create(ctx, n, descs, weights, act, x_offs, x_dtype, M, y_offs, fuse, specs, out);
     int per_cu = 0;
@@ -2583,6 +2718,8 @@ int ql_seq_run(ql_ctx* ctx, ql_seq* seq)
             case SeqStep::kPrefill: QL_HIP(ql::launch_prefill(st.p, true, ctx->stream)); break;
             case SeqStep::kGemm: QL_HIP(ql::launch_gemm_batch(st.gb, ctx->stream)); break;
             case SeqStep::kStrips: QL_HIP(ql::launch_strips(st.s, st.lds, ctx->stream)); break;
+            case SeqStep::kXImage: QL_HIP(ql::launch_x_image(st.xi, ctx->stream)); break;
+            case SeqStep::kGemvWave: QL_HIP(ql::launch_gemv_wave(st.gw, ctx->stream)); break;
             case SeqStep::kPartSums: QL_HIP(ql::launch_part_sums(st.sums, st.count, st.M, st.max_n, st.glu, ctx->stream)); break;
             }
         }

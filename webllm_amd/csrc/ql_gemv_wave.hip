@@ -105,7 +105,13 @@ __global__ __launch_bounds__(256) void x_image_kernel(const XImage a)
         return;
     }
     constexpr int KEEP = 2;                              // units a thread keeps: rows up to 4096 values
-    f32x4 v[KEEP][2];
+    f32x4 v[KEEP][2], gw[KEEP][2];                       // and their weights, loaded with them
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) {
+        const int u = min(tid + 256 * k, U - 1);
+        gw[k][0] = ld_global(reinterpret_cast<const f32x4*>(a.w) + 2 * u);
+        gw[k][1] = ld_global(reinterpret_cast<const f32x4*>(a.w) + 2 * u + 1);
+    }
     float ss = 0.f;
     auto add = [&](const f32x4& p, const f32x4& q) {
 #pragma unroll
@@ -127,28 +133,23 @@ __global__ __launch_bounds__(256) void x_image_kernel(const XImage a)
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
     const float rstd = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)a.K + a.eps);
-    for (int k = 0; k * 256 < U; k++) {
-        const int u = tid + 256 * k;
-        f32x4 p, q;
-        if (k == 0) {
-            p = v[0][0];
-            q = v[0][1];
-        } else if (k == 1) {
-            p = v[1][0];
-            q = v[1][1];
-        } else {
-            value(u, p, q);
-        }
-        if (u < U) {
-            const f32x4 g = ld_global(reinterpret_cast<const f32x4*>(a.w) + 2 * u), h = ld_global(reinterpret_cast<const f32x4*>(a.w) + 2 * u + 1);
+    auto norm = [&](int u, f32x4 p, f32x4 q, const f32x4& g, const f32x4& h) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                p[e] = p[e] * rstd * g[e];
-                q[e] = q[e] * rstd * h[e];
-            }
+        for (int e = 0; e < 4; e++) {
+            p[e] = p[e] * rstd * g[e];
+            q[e] = q[e] * rstd * h[e];
         }
-        if (!live) p = q = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!live || u >= U) p = q = f32x4{0.f, 0.f, 0.f, 0.f};
         put(u, p, q);
+    };
+#pragma unroll
+    for (int k = 0; k < KEEP; k++)
+        if (k * 256 < U) norm(tid + 256 * k, v[k][0], v[k][1], gw[k][0], gw[k][1]);
+    for (int k = KEEP; k * 256 < U; k++) {
+        const int u = tid + 256 * k, uu = min(u, U - 1);
+        f32x4 p, q;
+        value(u, p, q);
+        norm(u, p, q, ld_global(reinterpret_cast<const f32x4*>(a.w) + 2 * uu), ld_global(reinterpret_cast<const f32x4*>(a.w) + 2 * uu + 1));
     }
 }
 
