@@ -180,7 +180,7 @@ struct UnpackArgs {
 hipError_t launch_unpack(const UnpackArgs& a, bool fast, hipStream_t stream);
 // Batched fp16 unpack: up to kUnpackBatch tensors (each meeting the tile path's conditions: N % 4 == 0,
 // K % 8 == 0, 16-byte aligned qweight and output, 8-byte aligned scales) in one launch.
-constexpr int kUnpackBatch = 32;
+constexpr int kUnpackBatch = 84;    // kernel arguments stay within 4 KiB; a launch's start and tail cost about 3 us
 struct UnpackItem {
     const uint32_t* qweight;
     const uint32_t* qzeros;    // or nullptr (zero 8)
