@@ -1999,6 +1999,68 @@ bool prefill_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_a
 
 namespace {
 
+// Linears of some tens of rows (MFMA GEMM shapes, aligned) over fp16 images of x in the context's
+// workspace: one image per distinct x, then one launch. Returns false when it does not apply.
+bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
+               const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, int* rc)
+{
+    // Where it is the faster one, by its workgroups (64 columns x 32 rows): up to about a thousand with
+    // K <= 2048, where the other forms' K split and tiles cost more than the work (us, them -> this: 20 rows
+    // of 896 x 896 11.2 -> 6.9, 400 rows 10.6 -> 8.6; above a thousand the dequantization repeated per 32 rows
+    // tells: 256 rows of 896 -> 18944 19.0 -> 26.3); with a longer K from 160 workgroups on, because a
+    // wave's part of K is a serial chain (77 rows of 3584 x 3584 15.7 -> 12.7, 128 of 3584 -> 18944 43 -> 36, but
+    // 64 of 4864 -> 896 10.6 -> 14.6, 64 of 18944 -> 3584 27.5 -> 38.9).
+    long wgs = 0, n = 0;
+    int max_k = 0;
+    for (int i = 0; i < count; i++) {
+        if (descs[i].group % 128) return false;
+        wgs += (long)((descs[i].N + 63) / 64) * ((M + 31) / 32);
+        n += descs[i].N;
+        max_k = std::max(max_k, descs[i].K);
+    }
+    if (wgs > (max_k <= 2048 ? 1024 : 1200) || (max_k > 2048 && (wgs < 160 || n < 2048))) return false;
+    uint64_t off[ql::kMaxBatch], bytes = 0;
+    int first[ql::kMaxBatch];                               // the linear whose image linear i reads
+    for (int i = 0; i < count; i++) {
+        first[i] = i;
+        for (int k = i - 1; k >= 0; k--)
+            if (x_offs[k] == x_offs[i] && descs[k].K == descs[i].K) first[i] = k;
+        off[i] = first[i] < i ? off[first[i]] : bytes;
+        if (first[i] == i) bytes += align256(ql::x_rows_bytes(M, descs[i].K));
+    }
+    if (bytes > ql::kAttnTileWsBytes) return false;
+    if ((*rc = set_device(ctx))) return true;
+    char* ws = static_cast<char*>(ctx->tile_ws);
+    ql::FewBatch b{};
+    b.count = count;
+    b.M = M;
+    for (int i = 0; i < count; i++) {
+        const ql::GemvLinear g = make_linear(&descs[i], weights);
+        ql::FewLinear& L = b.L[i];
+        L.qweight = g.qweight;
+        L.qzeros = g.qzeros;
+        L.scales = g.scales;
+        L.bias = g.bias;
+        L.img = reinterpret_cast<decltype(L.img)>(ws + off[i]);
+        L.y = reinterpret_cast<float*>(act->base + y_offs[i]);
+        L.N = descs[i].N;
+        L.K = descs[i].K;
+        L.group = descs[i].group;
+    }
+    std::lock_guard<std::mutex> guard(ctx->ws_lock);
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < count && e == hipSuccess; i++)
+        if (first[i] == i)
+            e = ql::launch_x_rows(act->base + x_offs[i], x_dtype == QL_DTYPE_F32, ws + off[i], M, descs[i].K, ctx->stream);
+    if (e == hipSuccess) e = ql::launch_gemm_few(b, ctx->stream);
+    *rc = e == hipSuccess ? QL_OK : hip_fail(e, "launch_gemm_few");
+    return true;
+}
+
+}  // namespace
+
+namespace {
+
 // Decode linears (M <= 16, checked and aligned) over images of x in the context's workspace: one image
 // per distinct x, then one launch. Returns false when it does not apply.
 bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
@@ -2097,6 +2159,7 @@ int linear_impl(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_
         return QL_OK;
     }
     if (p.kind == QL_KIND_GEMM_MFMA && gemv_aligned(d, x_off, y_off)) {
+        if (few_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, &rc)) return rc;
         if (prefill_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, &rc)) return rc;
         ql::GemmBatch b{};
         int rc2 = gemm_entry(d, weights, act, x_off, M, y_off, partial, ctx->counters, 0, 0, &b.L[0], false);
@@ -2426,6 +2489,7 @@ int ql_linear_batch(ql_ctx* ctx, int32_t count, const ql_gptq_desc* descs,
             bm = b;
         }
     }
+    if (gemm && few_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, &rc)) return rc;
     if (gemm && prefill_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, &rc)) return rc;
     if (gemm) {
         // one launch; each linear's partial sums at its own offset, as ql_plan_batch sized them

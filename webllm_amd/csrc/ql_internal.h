@@ -119,6 +119,25 @@ GemmShape gemm_shape(int M, int N, int K, int group, int cu_count);
 uint64_t gemm_partial_bytes(int M, int N, int split);
 hipError_t launch_gemm_batch(const GemmBatch& b, hipStream_t stream);
 
+// GEMM of some tens of rows over fp16 images of x (ql_gemm_few.hip): gemm_fast_ok shapes with groups of a
+// multiple of 128, up to kMaxBatch linears on one M; launch_gemm_few fills wg_begin, wg_total and mb.
+struct FewLinear {
+    const uint32_t* qweight;
+    const uint32_t* qzeros;
+    const uint16_t* scales;
+    const float* bias;
+    const uint32_t __attribute__((ext_vector_type(4)))* img;   // x_rows_bytes(M, K)
+    float* y;
+    int N, K, group, wg_begin;
+};
+struct FewBatch {
+    FewLinear L[kMaxBatch];
+    int count, M, mb, wg_total;
+};
+uint64_t x_rows_bytes(int M, int K);
+hipError_t launch_x_rows(const void* x, bool f32, void* img, int M, int K, hipStream_t stream);
+hipError_t launch_gemm_few(FewBatch& b, hipStream_t stream);
+
 // Prefill GEMM over many linears in one persistent launch (M > 16, fp16 x, groups a multiple of
 // 128): tasks of one 128 x 256 output tile over all of K, from a host plan (table) or from the
 // tile numbering of a batch of up to kMaxBatch linears.
