@@ -59,6 +59,7 @@ struct SeqStep {
     const float* g = nullptr;
     const float* u = nullptr;
     float* o = nullptr;
+    bool half = false;                   // kGlu: o is fp16
     long long n = 0;
     ql::StripArgs s{};
     uint64_t lds = 0;
@@ -1130,6 +1131,8 @@ struct PrefillPasses {
     std::vector<char> chunked;                   // per pass: the chunked split-K GEMM
     std::vector<int> chunk_tiles;                // per chunked pass: its output tiles
     std::vector<char> deferred;                  // per chunked pass: a part-sum launch follows it
+    std::vector<char> half_pass;                 // per pass: its inputs are all fused ones, held in fp16
+    std::vector<char> half_input;                // per input: in fp16 (every pass that reads it is such)
     std::vector<char> folded;                    // per input: a SiLU-mul that its gate and up
                                                  // linears' part-sum launch writes
     uint64_t input_bytes = 0;
@@ -1223,6 +1226,26 @@ void plan_prefill_passes(const std::vector<ql::SeqSpec>& specs, const ql_seq_fus
                     if (ql::gemm_shape(M, sp.N, sp.K, sp.group, ql::kPlanCUs).split >= QL_GEMM_DEFER_SPLIT) P->deferred[p] = 1;
         } else {
             ql::plan_prefill(prefill_specs(sub), M, grid, &P->plans[p]);
+        }
+    }
+    // The GEMMs round fp32 activations to fp16 as they stage them, in every column tile. A pass whose inputs
+    // are all written by launches of the sequence gets them rounded there instead: the same values in half
+    // the bytes, and the GEMMs' fp16 forms (same K order, so the same sums to the bit).
+    P->half_pass.assign(P->depth, 1);
+    for (int i = 0; i < n; i++)
+        if (P->input_of[i] < 0 || specs[i].group % 128) P->half_pass[P->pass[i]] = 0;
+    P->half_input.assign(P->inputs.size(), 1);
+    for (bool again = true; again;) {
+        again = false;
+        for (int i = 0; i < n; i++) {
+            const int k = P->input_of[i];
+            if (k < 0) continue;
+            char& h = P->half_input[k];
+            char& hp = P->half_pass[P->pass[i]];
+            if (h != hp) {
+                h = hp = 0;
+                again = true;
+            }
         }
     }
     // a SiLU-mul of a gate and an up linear whose sums one part-sum launch adds (one pass, both
@@ -1444,12 +1467,14 @@ int prefill_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, con
                 st.g = ext_ptr(in.x_src, in.x_off);
                 st.u = ext_ptr(in.x2_src, in.x2_off);
                 st.o = buf;
+                st.half = P.half_input[k];
                 st.n = (long long)M * in.K;
             } else {
                 st.kind = SeqStep::kNorm;
                 st.e.x = ext_ptr(in.x_src, in.x_off);
                 st.e.w = reinterpret_cast<const float*>(weights->base + in.w_off);
                 st.e.y = buf;
+                if (P.half_input[k]) st.e.y16 = reinterpret_cast<uint16_t*>(buf);
                 st.e.M = M;
                 st.e.C = in.K;
                 st.e.eps = in.eps;
@@ -1473,7 +1498,7 @@ int prefill_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, con
             ql::GemmBatch& b = st.gb;
             b.count = (int)mem.size();
             b.M = M;
-            b.x_dtype = QL_DTYPE_F32;
+            b.x_dtype = P.half_pass[p] ? QL_DTYPE_F16 : QL_DTYPE_F32;
             long tiles = 0;
             for (int i : mem) {
                 const ql::GemmShape g = ql::gemm_shape(M, descs[i].N, descs[i].K, descs[i].group, ql::kPlanCUs);
@@ -1531,6 +1556,7 @@ int prefill_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, con
                 e.bias_b = sums[iu].bias;
                 e.yb = sums[iu].y;
                 e.yglu = reinterpret_cast<float*>(q->dev + P.inputs[k].buf_off);
+                e.glu_half = P.half_input[k];
                 drop[iu] = 1;
                 made[k] = true;
             }
@@ -1599,7 +1625,7 @@ int prefill_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, con
         st.p.task_begin = reinterpret_cast<const int32_t*>(dev + lay.task_begin);
         st.p.M = M;
         st.p.G = pp.grid;
-        st.p.x_f32 = 1;
+        st.p.x_f32 = !P.half_pass[p];
         q->steps.push_back(st);
     }
     fill_prefill_passes_info(P, n, prefill_passes_bytes(P), &q->info);
@@ -2441,7 +2467,7 @@ int ql_silu_mul(ql_ctx* ctx, ql_arena* act, uint64_t gate_off, uint64_t up_off, 
     if (rc) return rc;
     QL_HIP(ql::launch_silu_mul(reinterpret_cast<const float*>(act->base + gate_off),
                                reinterpret_cast<const float*>(act->base + up_off),
-                               reinterpret_cast<float*>(act->base + y_off), n, ctx->stream));
+                               reinterpret_cast<float*>(act->base + y_off), n, false, ctx->stream));
     return QL_OK;
 }
 
@@ -2778,7 +2804,7 @@ int ql_seq_run(ql_ctx* ctx, ql_seq* seq)
         for (const SeqStep& st : seq->steps) {
             switch (st.kind) {
             case SeqStep::kNorm: QL_HIP(ql::launch_add_rmsnorm(st.e, ctx->stream)); break;
-            case SeqStep::kGlu: QL_HIP(ql::launch_silu_mul(st.g, st.u, st.o, st.n, ctx->stream)); break;
+            case SeqStep::kGlu: QL_HIP(ql::launch_silu_mul(st.g, st.u, st.o, st.n, st.half, ctx->stream)); break;
             case SeqStep::kPrefill: QL_HIP(ql::launch_prefill(st.p, true, ctx->stream)); break;
             case SeqStep::kGemm: QL_HIP(ql::launch_gemm_batch(st.gb, ctx->stream)); break;
             case SeqStep::kStrips: QL_HIP(ql::launch_strips(st.s, st.lds, ctx->stream)); break;

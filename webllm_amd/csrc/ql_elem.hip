@@ -26,6 +26,15 @@ namespace {
 
 constexpr int kKeep = 4;     // 16-byte pieces of a row kept per thread: rows up to 4096 values
 
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+
+// four values of a result, as fp32 or (half) rounded to fp16
+__device__ __forceinline__ void st_result(float* y, uint16_t* y16, size_t i4, f32x4 v)
+{
+    if (y16) st_global(reinterpret_cast<f16x4*>(y16) + i4, __builtin_convertvector(v, f16x4));
+    else st_global(reinterpret_cast<f32x4*>(y) + i4, v);
+}
+
 __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const ElemArgs a)
 {
     __shared__ float red[4];
@@ -34,6 +43,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const ElemArgs a)
     const float* d = a.d ? a.d + (size_t)row * C : nullptr;
     float* s_out = a.s ? a.s + (size_t)row * C : nullptr;
     float* y = a.y + (size_t)row * C;
+    uint16_t* y16 = a.y16 ? a.y16 + (size_t)row * C : nullptr;
     float ss = 0.f;
     if (a.vec && C <= 4 * 256 * kKeep) {
         // one pass over HBM: the row (and the weight) stay in registers across the reduction
@@ -64,8 +74,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const ElemArgs a)
         for (int k = 0; k < kKeep; k++) {
             const int i = threadIdx.x + 256 * k;
             if (i < C / 4)
-                st_global(reinterpret_cast<f32x4*>(y) + i, f32x4{v[k].x * rstd * g[k].x, v[k].y * rstd * g[k].y,
-                                                                 v[k].z * rstd * g[k].z, v[k].w * rstd * g[k].w});
+                st_result(y, y16, i, f32x4{v[k].x * rstd * g[k].x, v[k].y * rstd * g[k].y, v[k].z * rstd * g[k].z, v[k].w * rstd * g[k].w});
         }
         return;
     }
@@ -114,8 +123,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const ElemArgs a)
                 }
             }
             const f32x4 g = ld_global(reinterpret_cast<const f32x4*>(a.w) + i);
-            st_global(reinterpret_cast<f32x4*>(y) + i,
-                      f32x4{v.x * rstd * g.x, v.y * rstd * g.y, v.z * rstd * g.z, v.w * rstd * g.w});
+            st_result(y, y16, i, f32x4{v.x * rstd * g.x, v.y * rstd * g.y, v.z * rstd * g.z, v.w * rstd * g.w});
         }
     } else {
         for (int i = threadIdx.x; i < C; i += 256) {
@@ -126,23 +134,28 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const ElemArgs a)
                 v = x[i];
                 if (d) v = v + d[i];
             }
-            y[i] = v * rstd * a.w[i];
+            const float r = v * rstd * a.w[i];
+            if (y16) y16[i] = __builtin_bit_cast(uint16_t, (_Float16)r);
+            else y[i] = r;
         }
     }
 }
 
 __device__ __forceinline__ float silu_mul1(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
-__global__ __launch_bounds__(256) void silu_mul_kernel(const float* gate, const float* up, float* y, long long n)
+// HALF: y fp16, n % 4 == 0
+template <bool HALF>
+__global__ __launch_bounds__(256) void silu_mul_kernel(const float* gate, const float* up, void* yv, long long n)
 {
+    float* y = static_cast<float*>(yv);
     const long long i4 = (long long)blockIdx.x * 256 + threadIdx.x;
     const long long n4 = n / 4;
     if (i4 < n4) {
         const f32x4 g = ld_global(reinterpret_cast<const f32x4*>(gate) + i4);
         const f32x4 u = ld_global(reinterpret_cast<const f32x4*>(up) + i4);
-        st_global(reinterpret_cast<f32x4*>(y) + i4,
+        st_result(y, HALF ? static_cast<uint16_t*>(yv) : nullptr, i4,
                   f32x4{silu_mul1(g.x, u.x), silu_mul1(g.y, u.y), silu_mul1(g.z, u.z), silu_mul1(g.w, u.w)});
-    } else if (i4 - n4 < n - 4 * n4) {
+    } else if (!HALF && i4 - n4 < n - 4 * n4) {
         const long long i = 4 * n4 + (i4 - n4);              // the tail (n % 4 values)
         y[i] = silu_mul1(gate[i], up[i]);
     }
@@ -156,10 +169,13 @@ hipError_t launch_add_rmsnorm(const ElemArgs& a, hipStream_t stream)
     return hipGetLastError();
 }
 
-hipError_t launch_silu_mul(const float* gate, const float* up, float* y, long long n, hipStream_t stream)
+hipError_t launch_silu_mul(const float* gate, const float* up, void* y, long long n, bool half, hipStream_t stream)
 {
+    if (half && n % 4) return hipErrorInvalidValue;
     const long long threads = n / 4 + (n % 4);
-    hipLaunchKernelGGL(silu_mul_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, gate, up, y, n);
+    const dim3 grid((unsigned)((threads + 255) / 256));
+    if (half) hipLaunchKernelGGL(silu_mul_kernel<true>, grid, dim3(256), 0, stream, gate, up, y, n);
+    else hipLaunchKernelGGL(silu_mul_kernel<false>, grid, dim3(256), 0, stream, gate, up, y, n);
     return hipGetLastError();
 }
 

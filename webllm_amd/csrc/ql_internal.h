@@ -268,12 +268,14 @@ struct ElemArgs {
     const float* w;            // [C] norm weight
     float* s;                  // x + d stored here (nullptr: not stored)
     float* y;                  // [M, C]
+    uint16_t* y16;             // set: the result rounded to fp16 goes here instead of y
     int M, C;
     float eps;
     int vec;                   // C % 4 == 0 and every pointer 16-byte aligned: f32x4 path
 };
 hipError_t launch_add_rmsnorm(const ElemArgs& a, hipStream_t stream);
-hipError_t launch_silu_mul(const float* gate, const float* up, float* y, long long n, hipStream_t stream);
+// half: y is fp16 (each value rounded to it), n a multiple of 4
+hipError_t launch_silu_mul(const float* gate, const float* up, void* y, long long n, bool half, hipStream_t stream);
 // Many rows (ql_attn_tile.hip): whether this call takes the tiled form within ws_bytes of workspace,
 // and its key splits
 constexpr size_t kAttnTileWsBytes = 64u << 20;
@@ -481,6 +483,7 @@ struct PartSum {
     const float* bias_b;
     float* yb;
     float* yglu;               // null: an ordinary entry (set in every entry of a glu launch)
+    int32_t glu_half;          // yglu is fp16
 };
 hipError_t launch_part_sums(const PartSum* entries_dev, int count, int M, int max_n, bool glu, hipStream_t stream);
 struct PartSumArgs {

@@ -893,8 +893,10 @@ __device__ __forceinline__ void part_sum_glu_entry(const PartSum& e, int M)
     if (r == 0) {
         st_global(reinterpret_cast<f32x4*>(e.y + o), t);
         st_global(reinterpret_cast<f32x4*>(e.yb + o), u);
-        st_global(reinterpret_cast<f32x4*>(e.yglu + o),
-                  f32x4{silu_mul1(t.x, u.x), silu_mul1(t.y, u.y), silu_mul1(t.z, u.z), silu_mul1(t.w, u.w)});
+        const f32x4 g = {silu_mul1(t.x, u.x), silu_mul1(t.y, u.y), silu_mul1(t.z, u.z), silu_mul1(t.w, u.w)};
+        typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+        if (e.glu_half) st_global(reinterpret_cast<f16x4*>(reinterpret_cast<uint16_t*>(e.yglu) + o), __builtin_convertvector(g, f16x4));
+        else st_global(reinterpret_cast<f32x4*>(e.yglu + o), g);
     }
 }
 
