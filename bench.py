@@ -394,7 +394,7 @@ def unpack_all(ctx, model: Model, steps: int):
     out_offs = [offs[k] for k in keys]
 
     def issue():
-        # the whole weight set through the batched entry point (six launches of 28 tensors)
+        # the whole weight set through the batched entry point (a few launches of up to 84 tensors)
         ctx.unpack_f16_batch(descs, model.arena, out, out_offs)
 
     issue()

@@ -1111,8 +1111,8 @@ int gemm_entry(const ql_gptq_desc* d, const ql_arena* weights, ql_arena* act, ui
 // the prefill kernel; a smaller one the chunked GEMM with K split across workgroups (the choice
 // ql_linear_batch makes), its partial sums and arrival counters in buffers of the sequence. A
 // fused RMSNorm or SiLU-mul input runs first, one launch per distinct input, into a buffer of the
-// sequence (fp32), as the reference runs its elementwise kernels between the GEMMs. Stream order
-// orders the passes.
+// sequence (fp32, or fp16 for passes that read nothing else: half_pass), as the reference runs its
+// elementwise kernels between the GEMMs. Stream order orders the passes.
 struct PrefillPasses {
     std::vector<int> pass;
     int depth = 0;
