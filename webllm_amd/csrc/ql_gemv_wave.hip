@@ -161,8 +161,8 @@ __device__ __forceinline__ float ror8(float v)           // the value of the lan
 // NT: 16-column tiles per wave; column n0 + NT i + t is tile t's row i, so a lane's words of a packed row
 // are adjacent. One group's loads at a time: 16 waves per CU hide them better than a ring in fewer waves
 // (two groups in flight, two waves per SIMD: 16.6 against 15.3 us at N = 18944, K = 3584, M = 8).
-template <int NT, bool BIG>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
+template <int NT, bool BIG, int W>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(W)))
 void gemv_wave_kernel(const GwBatch b)
 {
     static_assert(NT == 1 || NT == 4, "one word or one 16-byte load of a packed row per lane");
@@ -301,8 +301,11 @@ void gemv_wave_kernel(const GwBatch b)
 template <int NT>
 void launch_nt(const GwBatch& b, hipStream_t stream)
 {
-    if (b.M > 8) hipLaunchKernelGGL((gemv_wave_kernel<NT, true>), dim3(b.wg_total), dim3(512), 0, stream, b);
-    else hipLaunchKernelGGL((gemv_wave_kernel<NT, false>), dim3(b.wg_total), dim3(512), 0, stream, b);
+    if (b.M > 8) hipLaunchKernelGGL((gemv_wave_kernel<NT, true, 4>), dim3(b.wg_total), dim3(512), 0, stream, b);
+    // more workgroups than two per CU: fewer registers, so that a third fits (592 workgroups of 3584 -> 2 x 18944
+    // 22.1 -> 20.1 us, where they ran in two rounds; 296 of one of the two 14.5 -> 16.4)
+    else if (NT == 4 && b.wg_total > 2 * kPlanCUs) hipLaunchKernelGGL((gemv_wave_kernel<NT, false, 5>), dim3(b.wg_total), dim3(512), 0, stream, b);
+    else hipLaunchKernelGGL((gemv_wave_kernel<NT, false, 4>), dim3(b.wg_total), dim3(512), 0, stream, b);
 }
 
 }  // namespace
