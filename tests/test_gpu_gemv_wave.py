@@ -73,6 +73,7 @@ def run(ctx, M, shapes, x_dtype, same_x, biased, zeros, spread=False):
     (16, [(2048, 100)], ql.DTYPE_F16, False, False, "any", False),
     (16, [(256, 8228)], ql.DTYPE_F32, False, True, "any", False),        # 64-column tiles, ragged N
     (7, [(256, 8192)], ql.DTYPE_F16, False, False, "sym", False),
+    (8, [(128, 33000)], ql.DTYPE_F32, False, True, "any", False),        # 516 tiles: a third workgroup on some CUs
     (4, [(2048, 256)], ql.DTYPE_F32, False, True, "any", False),         # M = 3, 4: narrow, long K
     (3, [(4864, 896)], ql.DTYPE_F32, False, False, "any", False),
     (6, [(896, 896), (896, 128), (896, 128)], ql.DTYPE_F32, True, True, "any", False),     # one image for three
