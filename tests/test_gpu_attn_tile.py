@@ -93,3 +93,18 @@ def test_rows_do_not_see_later_keys_values(ctx):
     assert not np.isfinite(got[40:, :3, 7]).any() and close(got[40:80, :3, :7], clean[40:80, :3, :7])
     assert np.isnan(got[60:, 3:, 2]).all() and close(got[:, 3:, 3:], clean[:, 3:, 3:])
     assert np.isnan(got[80:, :3]).all()
+
+
+@pytest.mark.parametrize("keys", [slice(0, 1), slice(256, 257), slice(256, 384), slice(0, 1000)],
+                         ids=["first_key", "first_of_a_split", "a_whole_split", "all"])
+def test_nan_key_reaches_every_row_that_sees_it(ctx, keys):
+    """A NaN score makes its row NaN wherever the key lies: as the first key of all or of a key split (of 128 keys here),
+    where no other score has been seen yet, and where a split has no other."""
+    M, H, KV, D, past = 100, 6, 2, 64, 900
+    q, k, v = make(M, H, KV, D, past, 0xF1)
+    k[keys, 5] = np.nan                                       # of kv head 0
+    got = attend(ctx, q, k, v, past, 1024)
+    assert np.isnan(got[:, :3]).all()
+    from oracle import oracle as orc
+    clean = orc.attention_gqa_cache(q[:, 3:], np.ascontiguousarray(k[:, D:]), np.ascontiguousarray(v[:, D:]), 3, 1, D, past)
+    assert close(got[:, 3:], clean)

@@ -170,7 +170,7 @@ __device__ __forceinline__ void row_by_row(const AttnTile& a, int kvh, int r0, i
             for (int e = 0; e < E; e++) dot = fmaf(qv[e], a.k[off + 64 * e], dot);
             for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o);
             const float s = dot * a.scale, mn = fmaxf(mr, s);
-            if (mn == -INFINITY) continue;               // no visible key so far has a score above -inf
+            if (mr == -INFINITY && s == -INFINITY) continue;   // adds nothing yet; a NaN score (which fmaxf drops) stays
             const float c = ex2(mr - mn), p = ex2(s - mn);
             l = l * c + p;
             for (int e = 0; e < E; e++) acc[e] = fmaf(p, a.v[off + 64 * e], acc[e] * c);
