@@ -206,11 +206,13 @@ int ql_kv_store(ql_ctx* ctx, const ql_arena* act, uint64_t src_off, ql_arena* ca
 /* ql_attention_decode: out[m, h, :] = softmax_s(q[m, h] . K[s, h / (H / KV)] / sqrt(D)) V[s, ...]
  *   over s = 0 .. past_len + m (causal; attention/attention_gqa_cache.wgsl, CPU form
  *   reference/qwen-ref.ts:65-111 attentionGqaRef). q and out are [M, n_head, D] fp32 in `act`;
- *   D = 4..256 (multiple of 4); past_len + M <= max_t and <= 8192. fp32 throughout. Few rows x heads
- *   (decode) split the keys over workgroups, with partials in a 4 MiB workspace the context owns:
+ *   D = 4..256 (multiple of 4); past_len + M <= max_t and <= 8192. fp32 inputs, sums and results.
+ *   Few rows x heads (decode) split the keys over workgroups, with partials in a 4 MiB workspace the context owns:
  *   calls on one context run in its stream's order, so they never share it at the same time. Many rows
- *   (M >= 96 with past_len + M / 2 >= 896, D 64 or 128: prefill) run as tiles of 128 (row, head) pairs on
- *   the matrix cores, operands as two fp16 parts, with a 64 MiB workspace of the context's. */
+ *   (prefill: M >= 96, D 64 or 128, past_len + M / 2 at least 896 times the nsplit of ql_plan_attention) run as tiles
+ *   of 128 (row, head) pairs on the matrix cores, with a 64 MiB workspace of the context's: q, K, V and the
+ *   probabilities enter as two fp16 parts each (about 22 bits, no less exact than the other form's sums), in fp32
+ *   where their values lie too far apart for that. */
 int ql_attention_decode(ql_ctx* ctx, ql_arena* act, uint64_t q_off, const ql_arena* cache, uint64_t k_off,
                         uint64_t v_off, int32_t max_t, int32_t M, int32_t n_head, int32_t n_kv_head, int32_t D,
                         int32_t past_len, uint64_t out_off);

@@ -616,16 +616,17 @@ size_t image_bytes(int KV, int D, int blocks, int rows)
 }  // namespace
 
 // The line between this form and attn_kernel is where both its time and its error against 64 bits are the
-// smaller ones: at least 96 rows that see about 900 keys each on average. Measured (28 / 4 heads of 128; us
-// and relative error, attn_kernel -> this): 1024 rows after 1024 keys 630 -> 109, 2.5e-7 -> 2.1e-7; 128
-// after 1500 93 -> 38, 2.6e-7 -> 2.2e-7; 1024 after 400 416 -> 83, 2.2e-7 -> 2.0e-7. Beyond the line it is
-// mostly still faster but less exact, because attn_kernel's chains of fp32 sums are short there: 1024 rows
-// after none 247 -> 65 us but 1.4e-7 -> 1.5e-7; 48 after 2000 (which attn_kernel splits) 29 -> 20 us but
-// 1.9e-7 -> 2.1e-7 (14 / 2 heads of 64).
+// smaller ones: at least 96 rows that see about 900 keys each on average in every key split that attn_kernel
+// would take (a: planned; with few rows x heads it splits, and its chains of fp32 sums are then short). Measured (28 / 4
+// heads of 128; us and relative error, attn_kernel -> this): 1024 rows after 1024 keys 630 -> 110, 2.5e-7 ->
+// 2.1e-7; 128 after 1500 102 -> 41, 2.5e-7 -> 2.1e-7; 1024 after 400 417 -> 90, 2.15e-7 -> 2.0e-7. Beyond the
+// line it is mostly still faster but less exact: 1024 rows after none 247 -> 65 us but 1.4e-7 -> 1.5e-7; 14 / 2 heads
+// of 64, 96 rows after 912 (three splits) 1.78e-7 -> 1.89e-7, 160 after 880 (two) 1.97e-7 -> 1.99e-7; 28 / 4 of
+// 128, 96 after 848 (two) 57 -> 32 us but 1.85e-7 -> 1.89e-7.
 bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit)
 {
     if (a.D != 64 && a.D != 128) return false;
-    if (a.M < 96 || a.past + a.M / 2 < 896) return false;
+    if (a.M < 96 || a.past + a.M / 2 < 896 * a.nsplit) return false;
     const int blocks = (a.past + a.M + kBlk - 1) / kBlk;
     const int rows = (a.M * a.G + kRows - 1) / kRows;
     const size_t img = image_bytes(a.KV, a.D, blocks, rows);
