@@ -163,6 +163,8 @@ int ql_plan_linear(int32_t M, int32_t N, int32_t K, int32_t group, ql_plan* out)
 /* ---- y[M,N] (fp32) = x[M,K] * W^T (+ bias), enqueued on the context stream.
  * x_dtype: QL_DTYPE_F32 (decode path) or QL_DTYPE_F16. Offsets are into `act`.
  * scratch_off: plan.scratch_bytes bytes in `act` for split-K partial sums (ignored when 0).
+ * Images of x (M = 3..16 and prompts of some tens of rows, see ql_plan_linear) go through the context's 64 MiB
+ * workspace: calls on one context run in its stream's order.
  * The caller orders work by issuing it on this one stream (stream order replaces the
  * reference's passBreak, qwen.ts:556-559). */
 int ql_linear(ql_ctx* ctx, const ql_gptq_desc* desc, const ql_arena* weights, ql_arena* act,
@@ -372,7 +374,13 @@ int ql_sync(ql_ctx* ctx);
 int ql_timer_start(ql_ctx* ctx);
 int ql_timer_stop(ql_ctx* ctx, float* elapsed_ms); /* waits for the stop event */
 
-/* ---- stream capture into a HIP graph (one replayable submit per forward). */
+/* ---- stream capture into a HIP graph (one replayable submit per forward).
+ * A graph may be launched on any context of the device. Where its calls pass data through a workspace of the context
+ * (attention, ql_gemv_f16w, ql_linear and ql_linear_batch, as said there), it has one of its own, allocated while it
+ * is captured and freed with it, so it does not meet the context's other work. It does hold the capturing context's
+ * split-K arrival counters (ql_linear and ql_linear_batch with a plan that splits K): such a graph must not run
+ * beside that context's linears on another stream, nor outlive the context. ql_linear_noalloc allocates nothing:
+ * its captured launches use the static array, or the context's workspace where that is too small. */
 int ql_graph_begin(ql_ctx* ctx);
 int ql_graph_end(ql_ctx* ctx, ql_graph** out);
 int ql_graph_launch(ql_ctx* ctx, ql_graph* graph);

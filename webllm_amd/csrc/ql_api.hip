@@ -24,6 +24,7 @@ struct ql_ctx {
     void* tile_ws;        // ql::kAttnTileWsBytes, likewise: the many-row attention's images and partials
     std::mutex ws_lock;   // held while the launches that pass data through them are enqueued, so
                           // that another thread's do not come between them
+    std::vector<std::pair<void*, uint64_t>> graph_ws;   // during a capture: the graph's workspaces so far
     float* noalloc_scratch;  // this device's address of `scratch` (ql_linear_noalloc)
     hipEvent_t ev_start, ev_stop;
     bool capturing;
@@ -42,6 +43,7 @@ struct ql_arena {
 struct ql_graph {
     hipGraph_t graph;
     hipGraphExec_t exec;
+    std::vector<std::pair<void*, uint64_t>> ws;   // workspaces its launches use
 };
 
 // One launch of a pass-by-pass sequence: an RMSNorm into a buffer (e), a SiLU-mul into a buffer
@@ -114,6 +116,11 @@ int hip_fail(hipError_t e, const char* what)
 bool in_range(uint64_t off, uint64_t bytes, uint64_t size)
 {
     return off <= size && bytes <= size - off;
+}
+
+void free_workspaces(const std::vector<std::pair<void*, uint64_t>>& ws)
+{
+    for (const auto& w : ws) (void)hipFree(w.first);
 }
 
 uint64_t align256(uint64_t v) { return (v + 255) & ~(uint64_t)255; }
@@ -1684,6 +1691,7 @@ int ql_destroy(ql_ctx* ctx)
     (void)hipFree(ctx->counters);
     (void)hipFree(ctx->attn_ws);
     (void)hipFree(ctx->tile_ws);
+    free_workspaces(ctx->graph_ws);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return QL_OK;
@@ -2025,10 +2033,41 @@ bool prefill_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_a
 
 namespace {
 
-// Linears of some tens of rows (MFMA GEMM shapes, aligned) over fp16 images of x in the context's
+// Workspace of `bytes` for the launches enqueued now (ws_lock held): `own` (one of the context's, used in its
+// stream's order), or during a capture one that the graph keeps, because a graph may be launched on any
+// context's stream beside this one's work and may outlive the context. A graph's launches run in order, so they
+// share one unless a later one needs more.
+hipError_t workspace(ql_ctx* ctx, void* own, uint64_t bytes, void** out)
+{
+    *out = own;
+    if (!ctx->capturing || bytes == 0) return hipSuccess;
+    if (!ctx->graph_ws.empty() && ctx->graph_ws.back().second >= bytes) {
+        *out = ctx->graph_ws.back().first;
+        return hipSuccess;
+    }
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // an allocation does not enter the graph
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return e;
+    e = hipMalloc(out, bytes);
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return e;
+    ctx->graph_ws.emplace_back(*out, bytes);
+    return back;
+}
+
+// Where a linear's images of x go. `fixed` (ql_linear_noalloc, which allocates nothing): memory that a capture
+// uses where they fit instead of a workspace of the graph's.
+hipError_t image_workspace(ql_ctx* ctx, uint64_t bytes, void* fixed, void** out)
+{
+    if (!fixed) return workspace(ctx, ctx->tile_ws, bytes, out);
+    *out = ctx->capturing && bytes <= QL_NOALLOC_SCRATCH_BYTES ? fixed : ctx->tile_ws;
+    return hipSuccess;
+}
+
+// Linears of some tens of rows (MFMA GEMM shapes, aligned) over fp16 images of x in a
 // workspace: one image per distinct x, then one launch. Returns false when it does not apply.
 bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
-               const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, int* rc)
+               const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, void* fixed, int* rc)
 {
     // Where it is the faster one, by its workgroups (64 columns x 32 rows): up to about a thousand with
     // K <= 2048, where the other forms' K split and tiles cost more than the work (us, them -> this: 20 rows
@@ -2056,7 +2095,14 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
     }
     if (bytes > ql::kAttnTileWsBytes) return false;
     if ((*rc = set_device(ctx))) return true;
-    char* ws = static_cast<char*>(ctx->tile_ws);
+    std::lock_guard<std::mutex> guard(ctx->ws_lock);
+    void* base;
+    hipError_t e = image_workspace(ctx, bytes, fixed, &base);
+    if (e != hipSuccess) {
+        *rc = hip_fail(e, "image workspace");
+        return true;
+    }
+    char* ws = static_cast<char*>(base);
     ql::FewBatch b{};
     b.count = count;
     b.M = M;
@@ -2073,8 +2119,6 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
         L.K = descs[i].K;
         L.group = descs[i].group;
     }
-    std::lock_guard<std::mutex> guard(ctx->ws_lock);
-    hipError_t e = hipSuccess;
     for (int i = 0; i < count && e == hipSuccess; i++)
         if (first[i] == i)
             e = ql::launch_x_rows(act->base + x_offs[i], x_dtype == QL_DTYPE_F32, ws + off[i], M, descs[i].K, ctx->stream);
@@ -2087,10 +2131,10 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
 
 namespace {
 
-// Decode linears (M <= 16, checked and aligned) over images of x in the context's workspace: one image
+// Decode linears (M <= 16, checked and aligned) over images of x in a workspace: one image
 // per distinct x, then one launch. Returns false when it does not apply.
 bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
-                     const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, int* rc)
+                     const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, void* fixed, int* rc)
 {
     // Where it is the faster one: at M >= 5 everywhere (M = 8, us, gemv_mfma_kernel -> this: K = N = 896
     // 11.4 -> 8.0, 3584 x 3584 16.6 -> 7.9, 18944 -> 3584 28.8 -> 17.6, 3584 -> 2 x 18944 26.2 -> 22.2; M = 16
@@ -2116,7 +2160,14 @@ bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql
     }
     if (bytes > ql::kAttnTileWsBytes) return false;
     if ((*rc = set_device(ctx))) return true;
-    char* ws = static_cast<char*>(ctx->tile_ws);
+    std::lock_guard<std::mutex> guard(ctx->ws_lock);
+    void* base;
+    hipError_t e = image_workspace(ctx, bytes, fixed, &base);
+    if (e != hipSuccess) {
+        *rc = hip_fail(e, "image workspace");
+        return true;
+    }
+    char* ws = static_cast<char*>(base);
     ql::GwBatch b{};
     ql::XImage im[ql::kMaxBatch];
     b.count = count;
@@ -2131,8 +2182,6 @@ bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql
         b.L[i] = gw_linear(&descs[i], weights, im[i], reinterpret_cast<float*>(act->base + y_offs[i]), nullptr);
     }
     ql::gemv_wave_plan(&b, ctx->cu_count);
-    std::lock_guard<std::mutex> guard(ctx->ws_lock);
-    hipError_t e = hipSuccess;
     for (int i = 0; i < count && e == hipSuccess; i++)
         if (first[i] == i) e = ql::launch_x_image(im[i], ctx->stream);
     if (e == hipSuccess) e = ql::launch_gemv_wave(b, ctx->stream);
@@ -2151,10 +2200,10 @@ int ql_plan_linear(int32_t M, int32_t N, int32_t K, int32_t group, ql_plan* out)
 namespace {
 
 // ql_linear after its scratch has been resolved: `partial` holds the plan's scratch_bytes (split-K
-// partial sums; unused when the plan does not split K).
+// partial sums; unused when the plan does not split K); `fixed` as in image_workspace.
 int linear_impl(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_arena* act,
                 uint64_t x_off, int32_t x_dtype, int32_t M, uint64_t y_off, const ql_plan& p,
-                float* partial)
+                float* partial, void* fixed)
 {
     int rc;
     if ((rc = set_device(ctx))) return rc;
@@ -2163,7 +2212,7 @@ int linear_impl(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_
     L.y = reinterpret_cast<float*>(act->base + y_off);
 
     if (p.kind == QL_KIND_GEMV_MFMA && gemv_aligned(d, x_off, y_off)) {
-        if (gemv_wave_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, &rc)) return rc;
+        if (gemv_wave_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, fixed, &rc)) return rc;
         const ql::GemvShape s = ql::gemv_shape(M, d->N, d->K, d->group);
         ql::GemvBatch b{};
         L.split = s.split;
@@ -2185,7 +2234,7 @@ int linear_impl(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_
         return QL_OK;
     }
     if (p.kind == QL_KIND_GEMM_MFMA && gemv_aligned(d, x_off, y_off)) {
-        if (few_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, &rc)) return rc;
+        if (few_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, fixed, &rc)) return rc;
         if (prefill_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, &rc)) return rc;
         ql::GemmBatch b{};
         int rc2 = gemm_entry(d, weights, act, x_off, M, y_off, partial, ctx->counters, 0, 0, &b.L[0], false);
@@ -2238,7 +2287,7 @@ int ql_linear(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_ar
         if (scratch_off % 16) return fail(QL_E_ALIGN, "scratch offset must be 16-byte aligned");
     }
     return linear_impl(ctx, d, weights, act, x_off, x_dtype, M, y_off, p,
-                       reinterpret_cast<float*>(act->base + scratch_off));
+                       reinterpret_cast<float*>(act->base + scratch_off), nullptr);
 }
 
 int ql_linear_noalloc(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_arena* act,
@@ -2256,7 +2305,7 @@ int ql_linear_noalloc(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weight
                     "%u-byte static scratch (use ql_linear with a scratch offset)",
                     (unsigned long long)p.scratch_bytes, (unsigned)QL_NOALLOC_SCRATCH_BYTES);
     if (!ctx->noalloc_scratch) return fail(QL_E_STATE, "static scratch address not resolved");
-    return linear_impl(ctx, d, weights, act, x_off, x_dtype, M, y_off, p, ctx->noalloc_scratch);
+    return linear_impl(ctx, d, weights, act, x_off, x_dtype, M, y_off, p, ctx->noalloc_scratch, ctx->noalloc_scratch);
 }
 
 int ql_gemv_f16w(ql_ctx* ctx, const ql_arena* weights, uint64_t w_off, uint64_t bias_off,
@@ -2286,7 +2335,9 @@ int ql_gemv_f16w(ql_ctx* ctx, const ql_arena* weights, uint64_t w_off, uint64_t 
     a.N = N;
     a.K = K;
     std::lock_guard<std::mutex> guard(ctx->ws_lock);
-    QL_HIP(ql::launch_gemv_f16w(a, ql::gemv_f16w_fast_ok(M, N, K), ctx->cu_count, ctx->attn_ws, ql::kAttnWsBytes, ctx->stream));
+    void* ws;
+    QL_HIP(workspace(ctx, ctx->attn_ws, ql::gemv_f16w_uses_ws(M, K, ql::kAttnWsBytes) ? ql::kAttnWsBytes : 0, &ws));
+    QL_HIP(ql::launch_gemv_f16w(a, ql::gemv_f16w_fast_ok(M, N, K), ctx->cu_count, ws, ql::kAttnWsBytes, ctx->stream));
     return QL_OK;
 }
 
@@ -2397,7 +2448,6 @@ int ql_attention_decode(ql_ctx* ctx, ql_arena* act, uint64_t q_off, const ql_are
     a.k = reinterpret_cast<const float*>(cache->base + k_off);
     a.v = reinterpret_cast<const float*>(cache->base + v_off);
     a.out = reinterpret_cast<float*>(act->base + out_off);
-    a.ws = ctx->attn_ws;
     a.M = M;
     a.H = n_head;
     a.KV = n_kv_head;
@@ -2408,10 +2458,15 @@ int ql_attention_decode(ql_ctx* ctx, ql_arena* act, uint64_t q_off, const ql_are
     if (ql::plan_attention(&a)) return fail(QL_E_INVALID, "attention shape does not fit the workspace");
     std::lock_guard<std::mutex> guard(ctx->ws_lock);
     int tile_split;
-    if (ql::attention_tile_ok(a, ql::kAttnTileWsBytes, &tile_split)) {
-        QL_HIP(ql::launch_attention_tile(a, ctx->tile_ws, tile_split, ctx->stream));
+    uint64_t bytes;
+    void* ws;
+    if (ql::attention_tile_ok(a, ql::kAttnTileWsBytes, &tile_split, &bytes)) {
+        QL_HIP(workspace(ctx, ctx->tile_ws, bytes, &ws));
+        QL_HIP(ql::launch_attention_tile(a, ws, tile_split, ctx->stream));
         return QL_OK;
     }
+    QL_HIP(workspace(ctx, ctx->attn_ws, a.nsplit == 1 ? 0 : (uint64_t)M * n_head * a.nsplit * (D + 2) * sizeof(float), &ws));
+    a.ws = static_cast<float*>(ws);
     QL_HIP(ql::launch_attention(a, ctx->stream));
     return QL_OK;
 }
@@ -2515,7 +2570,7 @@ int ql_linear_batch(ql_ctx* ctx, int32_t count, const ql_gptq_desc* descs,
             bm = b;
         }
     }
-    if (gemm && few_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, &rc)) return rc;
+    if (gemm && few_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, nullptr, &rc)) return rc;
     if (gemm && prefill_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, &rc)) return rc;
     if (gemm) {
         // one launch; each linear's partial sums at its own offset, as ql_plan_batch sized them
@@ -2561,7 +2616,7 @@ int ql_linear_batch(ql_ctx* ctx, int32_t count, const ql_gptq_desc* descs,
         }
         return QL_OK;
     }
-    if (gemv_wave_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, &rc)) return rc;
+    if (gemv_wave_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, nullptr, &rc)) return rc;
     if ((rc = set_device(ctx))) return rc;
     ql::GemvBatch b{};
     b.count = count;
@@ -2902,17 +2957,25 @@ int ql_graph_end(ql_ctx* ctx, ql_graph** out)
     if (!ctx->capturing) return fail(QL_E_STATE, "no capture active");
     *out = nullptr;
     ctx->capturing = false;
+    std::vector<std::pair<void*, uint64_t>> ws;
+    ws.swap(ctx->graph_ws);
     hipGraph_t g = nullptr;
-    QL_HIP(hipStreamEndCapture(ctx->stream, &g));
+    hipError_t e = hipStreamEndCapture(ctx->stream, &g);
+    if (e != hipSuccess) {
+        free_workspaces(ws);
+        return hip_fail(e, "hipStreamEndCapture");
+    }
     hipGraphExec_t exec = nullptr;
-    hipError_t e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
     if (e != hipSuccess) {
         (void)hipGraphDestroy(g);
+        free_workspaces(ws);
         return hip_fail(e, "hipGraphInstantiate");
     }
     ql_graph* gr = new ql_graph();
     gr->graph = g;
     gr->exec = exec;
+    gr->ws.swap(ws);
     *out = gr;
     return QL_OK;
 }
@@ -2932,6 +2995,7 @@ int ql_graph_destroy(ql_graph* graph)
     if (!graph) return fail(QL_E_INVALID, "null graph");
     (void)hipGraphExecDestroy(graph->exec);
     (void)hipGraphDestroy(graph->graph);
+    free_workspaces(graph->ws);   // hipFree waits for outstanding work on the device
     delete graph;
     return QL_OK;
 }

@@ -623,7 +623,7 @@ size_t image_bytes(int KV, int D, int blocks, int rows)
 // line it is mostly still faster but less exact: 1024 rows after none 247 -> 65 us but 1.4e-7 -> 1.5e-7; 14 / 2 heads
 // of 64, 96 rows after 912 (three splits) 1.78e-7 -> 1.89e-7, 160 after 880 (two) 1.97e-7 -> 1.99e-7; 28 / 4 of
 // 128, 96 after 848 (two) 57 -> 32 us but 1.85e-7 -> 1.89e-7.
-bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit)
+bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit, uint64_t* used)
 {
     if (a.D != 64 && a.D != 128) return false;
     if (a.M < 96 || a.past + a.M / 2 < 896 * a.nsplit) return false;
@@ -637,6 +637,7 @@ bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit)
     int s = std::max(1, std::min(kWorkgroups / rb, (blocks + 1) / 2));
     const size_t one = (size_t)a.M * a.H * (a.D + 2) * sizeof(float);
     *nsplit = (int)std::min<size_t>(std::min(s, 128), std::max<size_t>(1, (ws_bytes - img) / one));
+    *used = img + (*nsplit > 1 ? *nsplit * one : 0);
     return true;
 }
 

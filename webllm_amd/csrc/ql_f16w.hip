@@ -372,16 +372,20 @@ static int gemv_f16w_mfma_rows(int K)
     return (int)std::min<size_t>(kMfRows, (kMfLdsMax - 16) / per_row);
 }
 
+// More rows than one pass takes (16, fewer where K is long: 4 at K = 3584): the tiled form reads the weights
+// once for all of them (M = 17 at 151936 x 896: 58 against 108 us in two passes; M = 5 at 32000 x 3584: 45
+// against 84 us). One row over is enough, its launch costs no more than a pass.
+bool gemv_f16w_uses_ws(int M, int K, size_t ws_bytes)
+{
+    return M > std::max(gemv_f16w_mfma_rows(K), 1) && K % 8 == 0 && gemm_f16w_rows(K, ws_bytes) >= 16;
+}
+
 hipError_t launch_gemv_f16w(const F16wArgs& a, bool fast, int cu_count, void* ws, size_t ws_bytes, hipStream_t stream)
 {
     // one row (the decode lm_head) keeps the fp32-FMA kernel, measured faster there; two or more
     // rows take the matrix-core form, which reads the weights once per 16 rows
     const int R = gemv_f16w_mfma_rows(a.K);
-    // more rows than one pass takes (16, fewer where K is long: 4 at K = 3584): the tiled form reads the
-    // weights once for all of them (M = 17 at 151936 x 896: 58 against 108 us in two passes; M = 5 at
-    // 32000 x 3584: 45 against 84 us). One row over is enough, its launch costs no more than a pass.
-    if (a.M > std::max(R, 1) && a.K % 8 == 0 && gemm_f16w_rows(a.K, ws_bytes) >= 16)
-        return launch_gemm_f16w(a, cu_count, ws, ws_bytes, stream);
+    if (gemv_f16w_uses_ws(a.M, a.K, ws_bytes)) return launch_gemm_f16w(a, cu_count, ws, ws_bytes, stream);
     if (R >= 1 && a.K % 8 == 0 && !(fast && a.M == 1)) {
         const int tiles = (a.N + 15) / 16;
         // resident workgroups (4 waves each, two per CU), each walking many tiles with x staged once

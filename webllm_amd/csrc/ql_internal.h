@@ -226,7 +226,9 @@ struct F16wArgs {
 };
 bool gemv_f16w_fast_ok(int M, int N, int K);
 size_t gemv_f16w_lds(int M, int K);
-// ws: a workspace for the many-row form's image of x, used in stream order
+// whether a call takes the many-row form, whose image of x needs a workspace (of up to ws_bytes)
+bool gemv_f16w_uses_ws(int M, int K, size_t ws_bytes);
+// ws: that workspace, used in stream order
 hipError_t launch_gemv_f16w(const F16wArgs& a, bool fast, int cu_count, void* ws, size_t ws_bytes, hipStream_t stream);
 // More rows than one pass of the GEMV (ql_f16w_gemm.hip): K % 8 == 0; gemm_f16w_rows gives the rows per
 // image that fit ws_bytes (below 16: K too long).
@@ -276,10 +278,10 @@ struct ElemArgs {
 hipError_t launch_add_rmsnorm(const ElemArgs& a, hipStream_t stream);
 // half: y is fp16 (each value rounded to it), n a multiple of 4
 hipError_t launch_silu_mul(const float* gate, const float* up, void* y, long long n, bool half, hipStream_t stream);
-// Many rows (ql_attn_tile.hip): whether this call takes the tiled form within ws_bytes of workspace,
-// and its key splits
+// Many rows (ql_attn_tile.hip): whether this call (planned by plan_attention) takes the tiled form within ws_bytes
+// of workspace, its key splits and the bytes of it that it uses
 constexpr size_t kAttnTileWsBytes = 64u << 20;
-bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit);
+bool attention_tile_ok(const AttnArgs& a, size_t ws_bytes, int* nsplit, uint64_t* used);
 hipError_t launch_attention_tile(const AttnArgs& a, void* ws, int nsplit, hipStream_t stream);
 hipError_t launch_attention(const AttnArgs& a, hipStream_t stream);
 hipError_t launch_kv_store(const float* src, float* dst, int rows, int row_len, int pos0, hipStream_t stream);
