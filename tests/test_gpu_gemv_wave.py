@@ -113,3 +113,61 @@ def test_replay_and_other_users_of_the_workspace(ctx):
     g.destroy()
     act.release()
     w.release()
+
+
+def test_widths_past_the_split_counters_stay_refused(ctx):
+    """256 x 65536 columns is the most that one call's arrival counters cover, whichever kernel runs."""
+    N = 256 * 65536 + 4
+    qw, qz, sc = ql.gptq_sizes(128, N, 128)
+    lay = ql.ArenaLayout()
+    d = ql.make_desc(lay.take(qw), None, lay.take(sc), 128, N, 128)
+    w = ctx.arena(lay.used)
+    for M in (4, 8):
+        alay = ql.ArenaLayout()
+        x, y = alay.take(M * 128 * 4), alay.take(M * N * 4)
+        scratch = alay.take(max(16, ql.plan_linear(M, N, 128).scratch_bytes))
+        act = ctx.arena(alay.used)
+        with pytest.raises(ql.QlError) as e:
+            ctx.linear(d, w, act, x, ql.DTYPE_F32, M, y, scratch)
+        assert e.value.code == -10 and "N too large" in str(e.value)
+        act.release()
+    # two linears of half as many columns and one strip more
+    half = ql.make_desc(d.qweight_off, None, d.scales_off, 128, 256 * 32768 + 4, 128)
+    alay = ql.ArenaLayout()
+    x, y = alay.take(8 * 128 * 4), [alay.take(8 * half.N * 4) for _ in range(2)]
+    scratch = alay.take(max(16, ql.plan_batch([half] * 2, 8)))
+    act = ctx.arena(alay.used)
+    with pytest.raises(ql.QlError) as e:
+        ctx.linear_batch([half] * 2, w, act, [x] * 2, ql.DTYPE_F32, 8, y, scratch)
+    assert e.value.code == -10 and "batch too wide" in str(e.value)
+    act.release()
+    w.release()
+
+
+def test_image_past_the_workspace(ctx):
+    """K so long that 16 rows' image outgrows the workspace's 64 MiB: the other decode kernel, at the same bar."""
+    M, K, N = 16, 128 * 8200, 64
+    g = np.random.default_rng(0x10A6)
+    qweight = g.integers(-2**31, 2**31, (K // 8, N), dtype=np.int64).astype(np.int32)
+    scales = (np.abs(g.standard_normal((K // 128, N))) * 0.01).astype(np.float16)
+    x = g.standard_normal((M, K)).astype(np.float32)
+    lay, alay = ql.ArenaLayout(), ql.ArenaLayout()
+    d = ql.make_desc(lay.take(qweight.nbytes), None, lay.take(scales.nbytes), K, N, 128)
+    w = ctx.arena(lay.used)
+    w.write(d.qweight_off, qweight)
+    w.write(d.scales_off, scales)
+    xo, yo = alay.take(x.nbytes), alay.take(M * N * 4)
+    scratch = alay.take(max(16, ql.plan_linear(M, N, K).scratch_bytes))
+    act = ctx.arena(alay.used)
+    act.write(xo, x)
+    ctx.linear(d, w, act, xo, ql.DTYPE_F32, M, yo, scratch)
+    y = act.read(yo, (M, N), np.float32)
+    ref = np.zeros((M, N))
+    for k in range(0, K, 128 * 200):
+        n = min(128 * 200, K - k)
+        q = (qweight[k // 8:(k + n) // 8, None, :] >> np.arange(0, 32, 4, dtype=np.int32)[None, :, None]) & 15
+        W = (q.reshape(n, N) - 8.0) * np.repeat(scales[k // 128:(k + n) // 128].astype(np.float64), 128, 0)
+        ref += x[:, k:k + n].astype(np.float64) @ W
+    assert np.linalg.norm(y - ref) <= 1e-5 * np.linalg.norm(ref)
+    act.release()
+    w.release()

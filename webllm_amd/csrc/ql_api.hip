@@ -2212,15 +2212,15 @@ int linear_impl(ql_ctx* ctx, const ql_gptq_desc* d, const ql_arena* weights, ql_
     L.y = reinterpret_cast<float*>(act->base + y_off);
 
     if (p.kind == QL_KIND_GEMV_MFMA && gemv_aligned(d, x_off, y_off)) {
-        if (gemv_wave_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, fixed, &rc)) return rc;
         const ql::GemvShape s = ql::gemv_shape(M, d->N, d->K, d->group);
+        if (s.strips > ql::kCounterCapacity) return fail(QL_E_INVALID, "N too large (%d)", d->N);
+        if (gemv_wave_batch(ctx, 1, d, weights, act, &x_off, x_dtype, M, &y_off, fixed, &rc)) return rc;
         ql::GemvBatch b{};
         L.split = s.split;
         L.strips = s.strips;
         L.wg_begin = 0;
         L.partial = partial;
         L.counters = ctx->counters;
-        if (s.strips > ql::kCounterCapacity) return fail(QL_E_INVALID, "N too large (%d)", d->N);
         b.L[0] = L;
         b.count = 1;
         b.M = M;
@@ -2616,6 +2616,9 @@ int ql_linear_batch(ql_ctx* ctx, int32_t count, const ql_gptq_desc* descs,
         }
         return QL_OK;
     }
+    int64_t strips = 0;
+    for (int i = 0; i < count; i++) strips += ql::gemv_shape(M, descs[i].N, descs[i].K, descs[i].group).strips;
+    if (strips > ql::kCounterCapacity) return fail(QL_E_INVALID, "batch too wide");
     if (gemv_wave_batch(ctx, count, descs, weights, act, x_offs, x_dtype, M, y_offs, nullptr, &rc)) return rc;
     if ((rc = set_device(ctx))) return rc;
     ql::GemvBatch b{};
@@ -2636,7 +2639,6 @@ int ql_linear_batch(ql_ctx* ctx, int32_t count, const ql_gptq_desc* descs,
         L.partial = reinterpret_cast<float*>(act->base + off);
         L.counters = ctx->counters + counter_base;
         counter_base += s.strips;
-        if (counter_base > ql::kCounterCapacity) return fail(QL_E_INVALID, "batch too wide");
         off += align256(ql::gemv_partial_bytes(M, d->N, s.split));
         wg += s.strips * s.split;
         b.L[i] = L;
