@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from tests.test_gpu_fused import FusedModel, _sample, check_fused
+from tests.test_gpu_seq import SeqModel, check_all
 from webllm_amd import qlinear as ql
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +50,50 @@ def test_image_passes_match_oracle(ctx, M, layers, C, I, KV):
 def test_small_passes_of_few_rows_keep_the_tiles(ctx, M, C, I, variant):
     m = FusedModel(ql, ctx, M, 1, C, I, 128)
     assert m.seq.info.variant == variant
+
+
+@pytest.mark.parametrize("M,layers,C,I,KV", [(5, 1, 896, 4864, 128), (8, 2, 896, 4864, 128), (16, 2, 896, 4864, 128), (16, 1, 3584, 18944, 512)])
+def test_fused_tiles_of_many_rows(ctx, monkeypatch, M, layers, C, I, KV):
+    """The dependency-ordered tiles at M >= 5, which chained sequences with other groups, fp16 x or QL_SEQ_PASSES=0 run."""
+    from oracle import oracle as orc
+    monkeypatch.setenv("QL_SEQ_PASSES", "0")
+    m = FusedModel(ql, ctx, M, layers, C, I, KV)
+    info = m.seq.info
+    assert info.kernel == ql.SEQ_TILES and info.variant == 0 and info.launches == 1
+    m.seq.run()
+    m.seq.status()
+    first = m.outputs()
+    check_fused(orc, m, first, f"tiles M={M} C={C}", **({"cols_for": _sample} if C == 3584 else {}))
+    m.seq.run()
+    m.seq.status()
+    assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(first, m.outputs()))
+    m.release()
+
+
+def test_chained_tiles_of_16_rows(ctx, monkeypatch):
+    """The same without fused work."""
+    from oracle import oracle as orc
+    monkeypatch.setenv("QL_SEQ_PASSES", "0")
+    m = SeqModel(ql, ctx, 16, layers=2, C=896, I=4864, KV=128)
+    assert m.seq.info.kernel == ql.SEQ_TILES and m.seq.info.variant == 0
+    m.seq.run()
+    m.seq.status()
+    check_all(orc, m, m.outputs(), "tiles M=16")
+    m.release()
+
+
+@pytest.mark.parametrize("env,variant", [("0", 0), ("1", 2)])
+def test_external_second_operand(ctx, monkeypatch, env, variant):
+    """test_fused_silu_mul_external_operand's sequence at M = 16, as tiles and over images."""
+    from oracle import oracle as orc
+    from tests.test_gpu_fused import test_fused_silu_mul_external_operand as check
+    monkeypatch.setenv("QL_SEQ_PASSES", env)
+    seen, run = [], ql.Seq.run
+
+    def noted(seq):
+        seen.append(seq.info.variant)
+        run(seq)
+
+    monkeypatch.setattr(ql.Seq, "run", noted)
+    check(ql, ctx, orc, 16)
+    assert seen == [variant]
