@@ -2069,12 +2069,16 @@ hipError_t image_workspace(ql_ctx* ctx, uint64_t bytes, void* fixed, void** out)
 bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
                const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, void* fixed, int* rc)
 {
-    // Where it is the faster one, by its workgroups (64 columns x 32 rows): up to about a thousand with
-    // K <= 2048, where the other forms' K split and tiles cost more than the work (us, them -> this: 20 rows
-    // of 896 x 896 11.2 -> 6.9, 400 rows 10.6 -> 8.6; above a thousand the dequantization repeated per 32 rows
-    // tells: 256 rows of 896 -> 18944 19.0 -> 26.3); with a longer K from 160 workgroups on, because a
-    // wave's part of K is a serial chain (77 rows of 3584 x 3584 15.7 -> 12.7, 128 of 3584 -> 18944 43 -> 36, but
-    // 64 of 4864 -> 896 10.6 -> 14.6, 64 of 18944 -> 3584 27.5 -> 38.9).
+    // Where it is the faster one, by its workgroups (64 columns x 32 rows), with weights that a cache holds and with
+    // weights that come from HBM (us, the other forms -> this, cached; HBM): up to about a thousand with K <= 2048,
+    // where the other forms' K split and tiles cost more than the work (20 rows of 896 x 896 11.0 -> 7.0; 7.7, 400
+    // rows 12.5 -> 8.2; 8.3; above a thousand the dequantization repeated per 32 rows tells: 256 rows of 896 -> 18944
+    // 19.0 -> 26.3). A wave's part of K is a serial chain, so a longer K needs more of them: from 160 on (77 rows of
+    // 3584 x 3584 17.3 -> 12.7; 17.7 -> 14.5, 64 of 3584 -> 5120 20.0 -> 12.3; 20.5 -> 14.1, 33 of 5504 -> 6144 17.3 ->
+    // 15.4; 18.7 -> 18.8, but 64 of 4864 -> 896 10.6 -> 14.6), and past 6144, where from HBM the chain takes about 2.2 us
+    // per 1024, 208 (128 rows of 18944 -> 3584 47.4 -> 40.5; 48.1 -> 47.9, but 77 45.2 -> 39.3; 45.5 -> 47.1), or 384 with
+    // two row tiles, which the other forms' 64 rows fit (33 of 18944 -> 13824 81 -> 57; 83 -> 75, but -> 10240
+    // 61 -> 57; 63 -> 73).
     long wgs = 0, n = 0;
     int max_k = 0;
     for (int i = 0; i < count; i++) {
@@ -2083,7 +2087,8 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
         n += descs[i].N;
         max_k = std::max(max_k, descs[i].K);
     }
-    if (wgs > (max_k <= 2048 ? 1024 : 1200) || (max_k > 2048 && (wgs < 160 || n < 2048))) return false;
+    const long least = max_k <= 6144 || M <= 32 ? 160 : M <= 64 ? 384 : 208;
+    if (wgs > (max_k <= 2048 ? 1024 : 1200) || (max_k > 2048 && (wgs < least || n < 2048))) return false;
     uint64_t off[ql::kMaxBatch], bytes = 0;
     int first[ql::kMaxBatch];                               // the linear whose image linear i reads
     for (int i = 0; i < count; i++) {
