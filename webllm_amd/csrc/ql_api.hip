@@ -2136,23 +2136,45 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
 
 namespace {
 
+// The longest K at which the products over images are the faster form for n columns in all, with weights that a cache
+// holds and with weights from HBM (as decode's are). A wave's part of K is a chain of groups whose loads
+// wait for each other, 1.1 us per 1024 of K where every CU has a workgroup at most (n <= 16 CUs), 2.1 to 3.4 above;
+// gemv_mfma_kernel's time grows with the rows instead. Measured (us, gemv_mfma_kernel -> this, cached; HBM), per band
+// of n on either side of its line:
+//   n <= 16 CUs: M = 3 8192 -> 4096 12.5 -> 9.1; 14.0 -> 13.2, 9472 -> 4096 12.5 -> 9.7; 14.2 -> 15.1; M = 5 11008 -> 4096
+//     17.2 -> 10.6; 18.6 -> 16.2, 18944 -> 4096 21.7 -> 16.5; 22.3 -> 24.3; M = 8 3584 -> 3584 16.6 -> 7.2; 17.5 -> 9.0,
+//     18944 -> 3584 28.8 -> 17.5; 30.4 -> 25.0; M = 9 (two fragments) 11008 -> 4096 24.0 -> 16.7; 25.6 -> 22.2, 18944 -> 4096
+//     31.6 -> 26.1; 32.2 -> 34.3
+//   to 20 CUs: M = 5 3584 -> 5120 14.0 -> 8.3; 15.6 -> 11.3, 6400 -> 5120 15.1 -> 10.7; 16.5 -> 17.1
+//   to 32 CUs: M = 4 3072 -> 8000 10.2 -> 8.1; 11.5 -> 10.8, 3584 -> 8000 10.1 -> 8.8; 11.4 -> 11.8; M = 8 6400 -> 8000
+//     17.7 -> 12.4; 19.2 -> 17.4, 11008 -> 8000 23.2 -> 18.2; 24.0 -> 25.4
+//   above: M = 5 2048 -> 10240 11.1 -> 8.0; 12.9 -> 10.9, 3584 -> 2 x 18944 22.5 -> 19.8; 25.1 -> 26.1; M = 8 3584 -> 2 x 18944
+//     26.2 -> 19.9; 29.2 -> 26.2, 11008 -> 10240 26.4 -> 24.3; 28.1 -> 33.4; M = 9 3584 -> 2 x 18944 37.1 -> 25.6;
+//     38.3 -> 34.2, 5760 -> 18816 29.2 -> 23.9; 30.6 -> 31.9
+// From 14 rows on it is faster throughout (M = 16 18944 -> 10240 83 -> 46; 85 -> 62).
+int gemv_wave_max_k(int M, long n, int cu_count)
+{
+    if (M >= 14) return INT32_MAX;
+    if (n <= 16L * cu_count) return (M <= 8 ? 2816 : 1792) * M;
+    if (n <= 20L * cu_count) return (M <= 8 ? 1200 : 768) * M;
+    return (n < 32L * cu_count ? 832 : M <= 8 ? 640 : 512) * M;
+}
+
 // Decode linears (M <= 16, checked and aligned) over images of x in a workspace: one image
 // per distinct x, then one launch. Returns false when it does not apply.
 bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
                      const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, void* fixed, int* rc)
 {
-    // Where it is the faster one: at M >= 5 everywhere (M = 8, us, gemv_mfma_kernel -> this: K = N = 896
-    // 11.4 -> 8.0, 3584 x 3584 16.6 -> 7.9, 18944 -> 3584 28.8 -> 17.6, 3584 -> 2 x 18944 26.2 -> 22.2; M = 16
-    // 18.4 -> 8.0, 27.6 -> 9.2, 52.8 -> 26.2, 49.4 -> 26.1), at M = 3, 4 for narrow linears with a long K, whose
-    // K split there costs round trips (M = 4: 3584 x 3584 11.7 -> 8.2, 3584 -> 2 x 18944 20.1 -> 20.7). At
-    // M = 1, 2 the image's launch costs more than it saves.
+    // At M = 1, 2 the image's launch costs more than it saves, at M = 3, 4 where there are many columns or K is short
+    // (M = 4: 3584 -> 2 x 18944 20.1 -> 20.7 us).
     long n = 0;
-    int min_k = INT32_MAX;
+    int min_k = INT32_MAX, max_k = 0;
     for (int i = 0; i < count; i++) {
         n += descs[i].N;
         min_k = std::min(min_k, descs[i].K);
+        max_k = std::max(max_k, descs[i].K);
     }
-    if (M < 3 || (M < 5 && (n >= 32L * ctx->cu_count || min_k < 2048))) return false;
+    if (M < 3 || (M < 5 && (n >= 32L * ctx->cu_count || min_k < 2048)) || max_k > gemv_wave_max_k(M, n, ctx->cu_count)) return false;
     uint64_t off[ql::kMaxBatch], bytes = 0;
     int first[ql::kMaxBatch];                               // the linear whose image linear i reads
     for (int i = 0; i < count; i++) {
