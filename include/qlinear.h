@@ -157,11 +157,22 @@ int ql_unpack_f32(ql_ctx* ctx, const ql_gptq_desc* desc, const ql_arena* weights
 int ql_unpack_f32_ex(ql_ctx* ctx, const ql_gptq_desc* desc, const ql_arena* weights, int32_t scales_dtype,
                      ql_arena* out, uint64_t out_off);
 
-/* ---- dispatch plan (host only, deterministic, pure). */
+/* ---- dispatch plan (host only, deterministic, pure): the kernel family, and the shape and scratch of its split-K
+ * form. scratch_bytes is what the caller has to provide (and what ql_linear_noalloc checks), an upper bound of what
+ * runs: where offsets are aligned, a call may take a kernel of the same family that splits nothing and leaves the
+ * scratch alone, which the plan does not tell because it depends on the offsets and the batch too:
+ *   M = 3..16, groups of 128, K up to a length that grows with M: products over an image of x (two launches; at 3 and
+ *     4 rows for K >= 2048 and few columns);
+ *   M > 16, groups a multiple of 128, up to about a thousand tiles of 64 columns x 32 rows (fewer where K is long):
+ *     the same over an fp16 image;
+ *   M > 16, enough tiles of 128 x 256: the prefill launch.
+ * ql_plan_batch likewise. */
 int ql_plan_linear(int32_t M, int32_t N, int32_t K, int32_t group, ql_plan* out);
 
 /* ---- y[M,N] (fp32) = x[M,K] * W^T (+ bias), enqueued on the context stream.
  * x_dtype: QL_DTYPE_F32 (decode path) or QL_DTYPE_F16. Offsets are into `act`.
+ * M <= 16: weights (q - zero) exact, fp16 scales, fp32 sums; x to 2^-30 of its group's largest value, or as two fp16
+ * parts of about 22 bits each (products over an image); fp16 weights and x rounded to fp16 above, as the reference.
  * scratch_off: plan.scratch_bytes bytes in `act` for split-K partial sums (ignored when 0).
  * Images of x (M = 3..16 and prompts of some tens of rows, see ql_plan_linear) go through the context's 64 MiB
  * workspace: calls on one context run in its stream's order.
@@ -190,7 +201,8 @@ int ql_linear_noalloc(ql_ctx* ctx, const ql_gptq_desc* desc, const ql_arena* wei
  * QwenGpt.gemm(lnf, 'embed', logits, null, M, V, C) (qwen.ts:488-489) on gemm_gemv_f16.wgsl's
  * arithmetic (fp32 x, fp16 weights, fp32 accumulation). M = 1..65535: up to 16 rows one pass over
  * the weights; more rows run as a tiled product that reads them once for up to about 1000 rows (K = 896), with
- * an image of x in the context's 4 MiB workspace (calls on one context run in its stream's order).
+ * an image of x in the context's 4 MiB workspace (calls on one context run in its stream's order). x is fp32 at
+ * M = 1, two scaled fp16 parts of about 22 bits above.
  * x, y, w offsets 16-byte aligned, K % 8 == 0. */
 int ql_gemv_f16w(ql_ctx* ctx, const ql_arena* weights, uint64_t w_off, uint64_t bias_off,
                  ql_arena* act, uint64_t x_off, int32_t M, int32_t N, int32_t K, uint64_t y_off);

@@ -1,5 +1,5 @@
-"""GPU: decode linears over an image of x (ql_linear and ql_linear_batch at M >= 5, and M = 3, 4 with a narrow N and a long
-K, groups of 128) against the oracle (double accumulation on the fp32-decoded weights) at the GEMV bar, at the edges of
+"""GPU: decode linears over an image of x (ql_linear and ql_linear_batch at M >= 5, and M = 3, 4 with a narrow N and K from
+2048 on, groups of 128, up to a longest K) against the oracle (double accumulation on the fp32-decoded weights) at the GEMV bar, at the edges of
 the kernel's tiles: 16 or 64 columns, 8 parts of K, 8 or 16 rows."""
 import numpy as np
 import pytest
@@ -171,3 +171,8 @@ def test_image_past_the_workspace(ctx):
     assert np.linalg.norm(y - ref) <= 1e-5 * np.linalg.norm(ref)
     act.release()
     w.release()
+
+
+@pytest.mark.parametrize("M,K", [(3, 8448), (3, 8576), (9, 16128), (9, 16256)])
+def test_both_sides_of_the_longest_k(ctx, M, K):
+    run(ctx, M, [(K, 68)], ql.DTYPE_F32, False, True, "any")

@@ -144,7 +144,7 @@ def test_unpack_all_168_tensors_05b(ql, ctx, orc):
         got = out.read(o, (t.N, t.K), np.uint16)
         wants.append(orc.dequantize_gptq_int4_f16(t.qweight, t.qzeros, t.scales, t.K, t.N, 128))
         assert np.array_equal(got, wants[i]), f"tensor {i} {linears[i]}"
-    # the batched entry point (the loader's whole weight set in six launches) into a cleared arena
+    # the batched entry point (the loader's whole weight set in a few launches) into a cleared arena
     out.release()
     out = ctx.arena(olay.used)
     out.write(0, np.full(olay.used // 2, 0xFFFF, np.uint16))

@@ -21,7 +21,8 @@ struct ql_ctx {
     uint32_t* counters;   // split-K arrival counters; every launch leaves them at zero
     float* attn_ws;       // ql::kAttnWsBytes, used in stream order: attention key-split partials, the
                           // many-row fp16 product's image of x
-    void* tile_ws;        // ql::kAttnTileWsBytes, likewise: the many-row attention's images and partials
+    void* tile_ws;        // ql::kAttnTileWsBytes, likewise: the many-row attention's images and partials,
+                          // the linears' images of x
     std::mutex ws_lock;   // held while the launches that pass data through them are enqueued, so
                           // that another thread's do not come between them
     std::vector<std::pair<void*, uint64_t>> graph_ws;   // during a capture: the graph's workspaces so far
@@ -2758,6 +2759,7 @@ int seq_create_impl(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, const ql_
     if (!fused && ql::strip_eligible(specs, M))
         return strip_create(ctx, n, descs, weights, act, x_offs, x_dtype, M, y_offs, specs, out);
     if (image_passes_ok(specs, fuse, M, x_dtype)) {
+        // the tiles' plan is made for its figures, and so that what it refuses stays refused
         ql_seq_info info;
         if ((rc = plan_seq_impl(n, descs, M, x_offs, x_dtype, y_offs, fuse, ctx->cu_count, &info))) return rc;
         return image_passes_create(ctx, n, descs, weights, act, x_offs, M, y_offs, fuse, specs, info, out);

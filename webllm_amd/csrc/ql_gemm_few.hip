@@ -10,8 +10,10 @@
 // fp16 part and the weights' scales in fp16. Nothing is split across workgroups, so there are no partial
 // sums in memory and no launch that adds them.
 //
-// What bounds it: latency (image, first loads, exchange) for small linears, then the vector work that
-// dequantizes 128 k x 64 columns (about 210 instructions for 32 MFMAs).
+// What bounds it: latency. A wave loads a 128-k chunk, waits and dequantizes it (about 210 vector instructions
+// for 32 MFMAs of 128 k x 64 columns), so its part of K is a serial chain, 1.8 us per 1024 of K with cached
+// weights and 2.2 from HBM. 77 rows of 3584 x 3584, 12.7 and 14.5 us: waves wait 57 % of their cycles, the VALU
+// is busy 26 % of the launch, the matrix cores 10 %.
 
 #include "ql_device.h"
 #include "ql_digits.h"

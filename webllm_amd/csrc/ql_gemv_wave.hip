@@ -17,8 +17,10 @@
 // order. Nothing is split across workgroups, so there are no arrival counters and no partial sums in
 // memory: their round trips were most of a small linear's time.
 //
-// What bounds it: latency (image, first loads, exchange) for small linears, HBM and L2 for large ones
-// (each workgroup reads the image: M <= 8 32 B, M > 8 64 B per k beside its 8 NT B of weights).
+// What bounds it: latency. Each wave loads a group, waits and computes, so its part of K is a serial chain
+// (gemv_wave_max_k says up to which K that is the faster way); each workgroup reads the image, M <= 8 32 B, M > 8
+// 64 B per k beside its 8 NT B of weights. 3584 -> 2 x 18944 at M = 8, 20 us: waves wait 74 % of their cycles,
+// the VALU is busy 42 % of the launch, the matrix cores 11 %.
 #include <algorithm>
 
 #include "ql_device.h"
