@@ -97,3 +97,18 @@ def test_external_second_operand(ctx, monkeypatch, env, variant):
     monkeypatch.setattr(ql.Seq, "run", noted)
     check(ql, ctx, orc, 16)
     assert seen == [variant]
+
+
+@pytest.mark.parametrize("M,K,N,variant", [(2, 8320, 4224, 0), (3, 8320, 4224, 0), (4, 8320, 4224, 2), (2, 8192, 4224, 2), (2, 8320, 4096, 2)])
+def test_deep_wide_passes_of_two_and_three_rows_keep_the_tiles(ctx, M, K, N, variant):
+    """N -> K -> N in two passes of 16 MiB and more: at 2 and 3 rows a K above 8192 needs one workgroup a CU at most."""
+    lay, alay = ql.ArenaLayout(), ql.ArenaLayout()
+    descs = [ql.make_desc(*[lay.take(b) for b in ql.gptq_sizes(k, n, 128)], k, n, 128) for k, n in ((N, K), (K, N))]
+    w = ctx.arena(lay.used)
+    x, h, y = alay.take(M * N * 4), alay.take(M * K * 4), alay.take(M * N * 4)
+    act = ctx.arena(alay.used)
+    seq = ctx.seq(descs, w, act, [x, h], ql.DTYPE_F32, M, [h, y])
+    assert seq.info.variant == variant and seq.info.kernel == ql.SEQ_TILES
+    seq.destroy()
+    act.release()
+    w.release()

@@ -1326,7 +1326,9 @@ uint64_t prefill_passes_bytes(const PrefillPasses& P)
 // little. Measured (us, tiles -> images): 24 layers of the small model (1.9 MB a pass) M = 4 777 -> 842,
 // M = 5 1080 -> 844, M = 8 1273 -> 845, M = 16 2561 -> 963; a layer of the large one (30 MB a pass) M = 2 79 -> 58,
 // M = 5 144 -> 59; between attentions (4 passes and one launch of its own) M = 1 88 -> 90, M = 2 95 -> 76,
-// M = 4 126 -> 77. Sequences that stream their weights from HBM keep the K-part strips (four layers of the
+// M = 4 126 -> 77; with weights from HBM M = 2 91 -> 84, M = 4 117 -> 85. At 2 and 3 rows a pass of a long K must fit a
+// workgroup a CU, or its waves' serial chains cost more from HBM than the tiles (40 heads of 128, 5120 -> 13824 -> 5120,
+// cached; HBM: M = 2 78 -> 78; 84 -> 106, M = 3 91 -> 78; 98 -> 106, M = 4 103 -> 78; 109 -> 107). Sequences that stream their weights from HBM keep the K-part strips (four layers of the
 // large model, M = 8 277 against 311).
 bool image_passes_ok(const std::vector<ql::SeqSpec>& specs, const ql_seq_fuse* fuse, int M, int32_t x_dtype)
 {
@@ -1339,8 +1341,15 @@ bool image_passes_ok(const std::vector<ql::SeqSpec>& specs, const ql_seq_fuse* f
         if ((specs[i].fuse & ql::kFuseNorm) && fuse[i].norm_w_off % 16) return false;
         bytes += specs[i].weight_bytes;
     }
+    if (M >= 5) return true;
     std::vector<int> pass;
-    return M >= 5 || bytes / std::max(1, seq_pass_of(specs, &pass)) >= (16u << 20);
+    const int depth = seq_pass_of(specs, &pass);
+    if (bytes / std::max(1, depth) < (16u << 20)) return false;
+    std::vector<long> n(depth, 0);
+    for (size_t i = 0; i < specs.size(); i++) n[pass[i]] += specs[i].N;
+    for (size_t i = 0; i < specs.size(); i++)
+        if (M <= 3 && specs[i].K > 8192 && n[pass[i]] > 16L * ql::kPlanCUs) return false;
+    return true;
 }
 
 // Per pass, an image of each distinct input (an RMSNorm, a SiLU-mul, or rows as they are), then the
