@@ -386,25 +386,18 @@ hipError_t launch_gemv_f16w(const F16wArgs& a, bool fast, int cu_count, void* ws
     // rows take the matrix-core form, which reads the weights once per 16 rows
     const int R = gemv_f16w_mfma_rows(a.K);
     if (gemv_f16w_uses_ws(a.M, a.K, ws_bytes)) return launch_gemm_f16w(a, cu_count, ws, ws_bytes, stream);
-    if (R >= 1 && a.K % 8 == 0 && !(fast && a.M == 1)) {
+    if (R >= 1 && a.M <= R && a.K % 8 == 0 && !(fast && a.M == 1)) {
         const int tiles = (a.N + 15) / 16;
         // resident workgroups (4 waves each, two per CU), each walking many tiles with x staged once
         const int grid = std::max(1, std::min((tiles + 3) / 4, 2 * cu_count));
-        for (int m0 = 0; m0 < a.M; m0 += R) {
-            F16wArgs p = a;
-            p.M = std::min(R, a.M - m0);
-            p.x = a.x + (size_t)m0 * a.K;
-            p.y = a.y + (size_t)m0 * a.N;
-            const size_t lds = gemv_f16w_mfma_lds(p.M, a.K);
-            const bool kfull = a.K % 32 == 0;
-            if (kfull && a.bias) hipLaunchKernelGGL((gemv_f16w_mfma_kernel<true, true>), dim3(grid), dim3(256), lds, stream, p);
-            else if (kfull) hipLaunchKernelGGL((gemv_f16w_mfma_kernel<true, false>), dim3(grid), dim3(256), lds, stream, p);
-            else if (a.bias) hipLaunchKernelGGL((gemv_f16w_mfma_kernel<false, true>), dim3(grid), dim3(256), lds, stream, p);
-            else hipLaunchKernelGGL((gemv_f16w_mfma_kernel<false, false>), dim3(grid), dim3(256), lds, stream, p);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
+        // one pass: more rows than R run in the tiled form (a K so long that its image does not fit has R = 0)
+        const size_t lds = gemv_f16w_mfma_lds(a.M, a.K);
+        const bool kfull = a.K % 32 == 0;
+        if (kfull && a.bias) hipLaunchKernelGGL((gemv_f16w_mfma_kernel<true, true>), dim3(grid), dim3(256), lds, stream, a);
+        else if (kfull) hipLaunchKernelGGL((gemv_f16w_mfma_kernel<true, false>), dim3(grid), dim3(256), lds, stream, a);
+        else if (a.bias) hipLaunchKernelGGL((gemv_f16w_mfma_kernel<false, true>), dim3(grid), dim3(256), lds, stream, a);
+        else hipLaunchKernelGGL((gemv_f16w_mfma_kernel<false, false>), dim3(grid), dim3(256), lds, stream, a);
+        return hipGetLastError();
     }
     if (!fast) {
         dim3 grid((a.N + 255) / 256, a.M);
