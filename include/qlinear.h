@@ -360,7 +360,8 @@ int ql_seq_status(ql_ctx* ctx, ql_seq* seq);
  * one launch before its pass. Stream order replaces the device-side waits (nothing can abort).
  * Other chained sequences (fused or not) with fp32 x, groups of 128, K % 128 == 0 and 16-byte aligned
  * norm weights run pass by pass over activation images at M = 5..16, and at M = 2..4 where a pass reads
- * 16 MiB of weights or more on average: per pass, one launch for each distinct input (an RMSNorm, a
+ * 16 MiB of weights or more on average (and, at 2 and 3 rows, a pass with K above 8192 has at most 4096
+ * columns): per pass, one launch for each distinct input (an RMSNorm, a
  * SiLU-mul, or rows as they are, as scaled fp16 parts) and one for the pass's linears. ql_plan_seq(_fused)
  * reports the tiles' plan for them, ql_seq_get_info variant 2 and the launches enqueued.
  * QL_SEQ_PASSES=0 in the environment keeps the tiles. */
