@@ -162,7 +162,7 @@ int ql_unpack_f32_ex(ql_ctx* ctx, const ql_gptq_desc* desc, const ql_arena* weig
  * runs: where offsets are aligned, a call may take a kernel of the same family that splits nothing and leaves the
  * scratch alone, which the plan does not tell because it depends on the offsets and the batch too:
  *   M = 3..16, groups of 128, K up to a length that grows with M: products over an image of x (two launches; at 3 and
- *     4 rows for K >= 2048 and few columns);
+ *     4 rows for K from 2304 and 2048 on and few columns);
  *   M > 16, groups a multiple of 128, up to about a thousand tiles of 64 columns x 32 rows (fewer where K is long):
  *     the same over an fp16 image;
  *   M > 16, enough tiles of 128 x 256: the prefill launch.
@@ -361,8 +361,8 @@ int ql_seq_status(ql_ctx* ctx, ql_seq* seq);
  * Other chained sequences (fused or not) with fp32 x, groups of 128, K % 128 == 0 and 16-byte aligned
  * norm weights run pass by pass over activation images at M = 5..16, and at M = 2..4 where a pass reads
  * 16 MiB of weights or more on average (and, at 2 and 3 rows, a pass with K above 8192 has at most 4096
- * columns): per pass, one launch for each distinct input (an RMSNorm, a
- * SiLU-mul, or rows as they are, as scaled fp16 parts) and one for the pass's linears. ql_plan_seq(_fused)
+ * columns): per pass, a launch for its distinct inputs of each kind (RMSNorms, SiLU-muls, rows as they are, as
+ * scaled fp16 parts) and one for its linears, up to eight inputs or linears a launch. ql_plan_seq(_fused)
  * reports the tiles' plan for them, ql_seq_get_info variant 2 and the launches enqueued.
  * QL_SEQ_PASSES=0 in the environment keeps the tiles. */
 typedef struct ql_seq_fuse {

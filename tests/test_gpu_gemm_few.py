@@ -81,3 +81,8 @@ def test_few_rows_match_fp16_operands(ctx, M, shapes, group, x_dtype, same_x, bi
     assert all(np.array_equal(a.view(np.uint32), c.view(np.uint32)) for a, c in zip(first, call()))
     act.release()
     w.release()
+
+
+def test_eight_inputs_of_a_batch(ctx):
+    """Eight linears on inputs of their own, of several K, images in one launch."""
+    test_few_rows_match_fp16_operands(ctx, 35, [(128 * (1 + 3 * (i % 3)), 64 + 4 * i) for i in range(8)], 128, ql.DTYPE_F32, False, True, "any")

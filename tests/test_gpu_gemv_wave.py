@@ -176,3 +176,9 @@ def test_image_past_the_workspace(ctx):
 @pytest.mark.parametrize("M,K", [(3, 8448), (3, 8576), (9, 16128), (9, 16256)])
 def test_both_sides_of_the_longest_k(ctx, M, K):
     run(ctx, M, [(K, 68)], ql.DTYPE_F32, False, True, "any")
+
+
+@pytest.mark.parametrize("M", [5, 16])
+def test_eight_inputs_of_a_batch(ctx, M):
+    """Eight linears on inputs of their own, of several K, images in one launch."""
+    run(ctx, M, [(128 * (1 + 3 * (i % 3)), 64 + 4 * i) for i in range(8)], ql.DTYPE_F32, False, True, "any")

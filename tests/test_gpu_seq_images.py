@@ -7,6 +7,7 @@ import pytest
 from tests.test_gpu_fused import FusedModel, _sample, check_fused
 from tests.test_gpu_seq import SeqModel, check_all
 from webllm_amd import qlinear as ql
+from webllm_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -109,6 +110,46 @@ def test_deep_wide_passes_of_two_and_three_rows_keep_the_tiles(ctx, M, K, N, var
     act = ctx.arena(alay.used)
     seq = ctx.seq(descs, w, act, [x, h], ql.DTYPE_F32, M, [h, y])
     assert seq.info.variant == variant and seq.info.kernel == ql.SEQ_TILES
+    seq.destroy()
+    act.release()
+    w.release()
+
+
+def test_inputs_of_a_pass_share_launches(ctx):
+    """Ten linears on inputs of their own and one on an RMSNorm in one pass, a twelfth on the first one's output: a launch
+    holds up to eight images of a kind."""
+    from oracle import oracle as orc
+    M, shapes = 6, [(256 if i % 2 else 384, 128 if i else 256) for i in range(10)] + [(640, 64), (256, 132)]
+    g = [synth.gptq_linear(K, N, 128, seed=0x5E7, key=(i,)) for i, (K, N) in enumerate(shapes)]
+    norm = 1 + 0.1 * synth.activations(1, 640, seed=0x5E8)[0]
+    lay, alay = ql.ArenaLayout(), ql.ArenaLayout()
+    offs = [[lay.take(a.nbytes) for a in (t.qweight, t.qzeros, t.scales)] for t in g]
+    norm_off = lay.take(norm.nbytes)
+    w = ctx.arena(lay.used)
+    for t, o in zip(g, offs):
+        for at, a in zip(o, (t.qweight, t.qzeros, t.scales)):
+            w.write(at, a)
+    w.write(norm_off, norm.astype(np.float32))
+    x = [synth.activations(M, K, seed=0x5E9, key=(i,)) for i, (K, N) in enumerate(shapes[:11])]
+    xo = [alay.take(a.nbytes) for a in x]
+    yo = [alay.take(M * N * 4) for _, N in shapes]
+    act = ctx.arena(alay.used)
+    for o, a in zip(xo, x):
+        act.write(o, a)
+    fuse = [ql.make_fuse(norm_w_off=norm_off if i == 10 else None) for i in range(12)]
+    descs = [ql.make_desc(*o, K, N, 128) for o, (K, N) in zip(offs, shapes)]
+    seq = ctx.seq(descs, w, act, xo + [yo[0]], ql.DTYPE_F32, M, yo, fuse=fuse)
+    assert seq.info.variant == 2 and seq.info.passes == 2
+    assert seq.info.launches == 2 + 1 + 2 + 1 + 1        # images (plain, norm), products; then one of each
+    for _ in range(2):
+        seq.run()
+        seq.status()
+    y = [act.read(o, (M, N), np.float32) for o, (_, N) in zip(yo, shapes)]
+    x[10] = orc.add_rmsnorm(x[10], norm.astype(np.float32), 1e-6)[1]
+    for t, a, b in zip(g, x + [y[0]], y):
+        ref = orc.gptq_linear(t.qweight, t.qzeros, t.scales, a, None, 128)
+        ok, ma, mr = orc.check_tolerance(b, ref, 1e-5 * max(1.0, float(np.sqrt(np.mean(a.astype(np.float64) ** 2)))), 1e-4)
+        assert ok, (ma, mr)
     seq.destroy()
     act.release()
     w.release()

@@ -53,7 +53,7 @@ struct ql_graph {
 // images (gw).
 struct SeqStep {
     enum Kind { kNorm, kGlu, kStrips, kPartSums, kPrefill, kGemm, kXImage, kGemvWave } kind;
-    ql::XImage xi{};
+    ql::XImageBatch xi{};
     ql::GwBatch gw{};
     const ql::PartSum* sums = nullptr;   // kPartSums: the device table, count entries
     int count = 0, M = 0, max_n = 0;
@@ -1352,8 +1352,8 @@ bool image_passes_ok(const std::vector<ql::SeqSpec>& specs, const ql_seq_fuse* f
     return true;
 }
 
-// Per pass, an image of each distinct input (an RMSNorm, a SiLU-mul, or rows as they are), then the
-// pass's products (launches of up to kMaxBatch linears), bias and residual at the store. The launches run
+// Per pass, images of its distinct inputs (a launch of up to kMaxBatch for its RMSNorms, one for its SiLU-muls, one
+// for rows as they are), then the pass's products (launches of up to kMaxBatch linears), bias and residual at the store. The launches run
 // in stream order; nothing waits on the device.
 int image_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
                         const uint64_t* x_offs, int32_t M, const uint64_t* y_offs, const ql_seq_fuse* fuse,
@@ -1410,13 +1410,19 @@ int image_passes_create(ql_ctx* ctx, int32_t n, const ql_gptq_desc* descs, const
     std::vector<bool> made(image.size(), false);
     for (int p = 0; p < P.depth; p++) {
         const std::vector<int>& mem = P.members[p];
+        const size_t first = q->steps.size();
         for (int i : mem) {
             if (made[image_of[i]]) continue;
             made[image_of[i]] = true;
-            SeqStep st{};
-            st.kind = SeqStep::kXImage;
-            st.xi = image[image_of[i]];
-            q->steps.push_back(st);
+            const ql::XImage& im = image[image_of[i]];
+            // into a launch of this pass for its kind, if one has room
+            size_t at = first;
+            while (at < q->steps.size() && (q->steps[at].xi.im[0].kind != im.kind || q->steps[at].xi.count == ql::kMaxBatch)) at++;
+            if (at == q->steps.size()) {
+                q->steps.emplace_back();
+                q->steps[at].kind = SeqStep::kXImage;
+            }
+            q->steps[at].xi.im[q->steps[at].xi.count++] = im;
         }
         for (size_t at = 0; at < mem.size(); at += ql::kMaxBatch) {
             SeqStep st{};
@@ -2075,7 +2081,7 @@ hipError_t image_workspace(ql_ctx* ctx, uint64_t bytes, void* fixed, void** out)
 }
 
 // Linears of some tens of rows (MFMA GEMM shapes, aligned) over fp16 images of x in a
-// workspace: one image per distinct x, then one launch. Returns false when it does not apply.
+// workspace: a launch for the images of the distinct x, then one. Returns false when it does not apply.
 bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
                const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, void* fixed, int* rc)
 {
@@ -2134,9 +2140,15 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
         L.K = descs[i].K;
         L.group = descs[i].group;
     }
-    for (int i = 0; i < count && e == hipSuccess; i++)
-        if (first[i] == i)
-            e = ql::launch_x_rows(act->base + x_offs[i], x_dtype == QL_DTYPE_F32, ws + off[i], M, descs[i].K, ctx->stream);
+    ql::XRows xr{};
+    xr.M = M;
+    for (int i = 0; i < count; i++)
+        if (first[i] == i) {
+            xr.x[xr.count] = act->base + x_offs[i];
+            xr.img[xr.count] = reinterpret_cast<decltype(xr.img[0] + 0)>(ws + off[i]);
+            xr.K[xr.count++] = descs[i].K;
+        }
+    e = ql::launch_x_rows(xr, x_dtype == QL_DTYPE_F32, ctx->stream);
     if (e == hipSuccess) e = ql::launch_gemm_few(b, ctx->stream);
     *rc = e == hipSuccess ? QL_OK : hip_fail(e, "launch_gemm_few");
     return true;
@@ -2170,8 +2182,8 @@ int gemv_wave_max_k(int M, long n, int cu_count)
     return (n < 32L * cu_count ? 832 : M <= 8 ? 640 : 512) * M;
 }
 
-// Decode linears (M <= 16, checked and aligned) over images of x in a workspace: one image
-// per distinct x, then one launch. Returns false when it does not apply.
+// Decode linears (M <= 16, checked and aligned) over images of x in a workspace: a launch for the
+// images of the distinct x, then one. Returns false when it does not apply.
 bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena* weights, ql_arena* act,
                      const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, void* fixed, int* rc)
 {
@@ -2206,21 +2218,24 @@ bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql
     }
     char* ws = static_cast<char*>(base);
     ql::GwBatch b{};
-    ql::XImage im[ql::kMaxBatch];
+    ql::XImageBatch im{};
     b.count = count;
     b.M = M;
+    const ql::XImage* made[ql::kMaxBatch];
     for (int i = 0; i < count; i++) {
-        im[i] = ql::XImage{};
-        im[i].x = act->base + x_offs[i];
-        im[i].M = M;
-        im[i].K = descs[i].K;
-        im[i].f16 = x_dtype == QL_DTYPE_F16;
-        ql::x_image_at(&im[i], ws + off[i]);
-        b.L[i] = gw_linear(&descs[i], weights, im[i], reinterpret_cast<float*>(act->base + y_offs[i]), nullptr);
+        if (first[i] == i) {
+            ql::XImage& x = im.im[im.count++];
+            x.x = act->base + x_offs[i];
+            x.M = M;
+            x.K = descs[i].K;
+            x.f16 = x_dtype == QL_DTYPE_F16;
+            ql::x_image_at(&x, ws + off[i]);
+            made[i] = &x;
+        }
+        b.L[i] = gw_linear(&descs[i], weights, *made[first[i]], reinterpret_cast<float*>(act->base + y_offs[i]), nullptr);
     }
     ql::gemv_wave_plan(&b, ctx->cu_count);
-    for (int i = 0; i < count && e == hipSuccess; i++)
-        if (first[i] == i) e = ql::launch_x_image(im[i], ctx->stream);
+    e = ql::launch_x_image(im, ctx->stream);
     if (e == hipSuccess) e = ql::launch_gemv_wave(b, ctx->stream);
     *rc = e == hipSuccess ? QL_OK : hip_fail(e, "launch_gemv_wave");
     return true;

@@ -27,7 +27,7 @@ __device__ const uint32_t kFewSymZeros = 0x77777777u;    // stored zeros of a li
 
 // x [M, K] (fp32, rounded to fp16, or fp16) -> image, a unit per thread; rows up to Mp are zero
 template <bool F32>
-__global__ __launch_bounds__(256) void x_rows_kernel(const void* x, u32x4* img, int M, int Mp, int K)
+__device__ __forceinline__ void x_rows(const void* x, u32x4* img, int M, int Mp, int K)
 {
     const int i = blockIdx.x * 256 + threadIdx.x, per = K / 8;
     if (i >= Mp * per) return;
@@ -48,6 +48,18 @@ __global__ __launch_bounds__(256) void x_rows_kernel(const void* x, u32x4* img, 
         }
     }
     st_global(img + ((size_t)(m >> 4) * (K / 32) + (u >> 2)) * 64 + (u & 3) * 16 + (m & 15), r);
+}
+
+// One input, whose few arguments are in registers when the wave starts (0.35 us less than from the struct), or several.
+template <bool F32>
+__global__ __launch_bounds__(256) void x_rows_kernel(const void* x, u32x4* img, int M, int Mp, int K)
+{
+    x_rows<F32>(x, img, M, Mp, K);
+}
+template <bool F32>
+__global__ __launch_bounds__(256) void x_rows_batch_kernel(const XRows a, int Mp)
+{
+    x_rows<F32>(a.x[blockIdx.y], a.img[blockIdx.y], a.M, Mp, a.K[blockIdx.y]);
 }
 
 // Two row tiles keep four waves per SIMD (114 registers), which hide the loads: three or four, in two waves
@@ -147,12 +159,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void g
 
 uint64_t x_rows_bytes(int M, int K) { return (uint64_t)((M + 16 * MT - 1) / (16 * MT) * (16 * MT)) * K * 2; }
 
-hipError_t launch_x_rows(const void* x, bool f32, void* img, int M, int K, hipStream_t stream)
+hipError_t launch_x_rows(const XRows& a, bool f32, hipStream_t stream)
 {
-    const int Mp = (M + 16 * MT - 1) / (16 * MT) * (16 * MT);
-    const dim3 grid(((unsigned)Mp * (K / 8) + 255) / 256);
-    if (f32) hipLaunchKernelGGL(x_rows_kernel<true>, grid, dim3(256), 0, stream, x, static_cast<u32x4*>(img), M, Mp, K);
-    else hipLaunchKernelGGL(x_rows_kernel<false>, grid, dim3(256), 0, stream, x, static_cast<u32x4*>(img), M, Mp, K);
+    if (a.count < 1 || a.count > kMaxBatch) return hipErrorInvalidValue;
+    const int Mp = (a.M + 16 * MT - 1) / (16 * MT) * (16 * MT);
+    int max_k = 0;
+    for (int i = 0; i < a.count; i++) max_k = a.K[i] > max_k ? a.K[i] : max_k;
+    const dim3 grid(((unsigned)Mp * (max_k / 8) + 255) / 256, a.count);
+    if (a.count == 1 && f32) hipLaunchKernelGGL(x_rows_kernel<true>, grid, dim3(256), 0, stream, a.x[0], a.img[0], a.M, Mp, a.K[0]);
+    else if (a.count == 1) hipLaunchKernelGGL(x_rows_kernel<false>, grid, dim3(256), 0, stream, a.x[0], a.img[0], a.M, Mp, a.K[0]);
+    else if (f32) hipLaunchKernelGGL(x_rows_batch_kernel<true>, grid, dim3(256), 0, stream, a, Mp);
+    else hipLaunchKernelGGL(x_rows_batch_kernel<false>, grid, dim3(256), 0, stream, a, Mp);
     return hipGetLastError();
 }
 

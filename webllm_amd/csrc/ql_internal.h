@@ -58,7 +58,12 @@ struct XImage {
 };
 uint64_t x_image_bytes(int M, int K);
 void x_image_at(XImage* a, void* p);
-hipError_t launch_x_image(const XImage& a, hipStream_t stream);
+// up to kMaxBatch images of one M, kind and f16 in one launch
+struct XImageBatch {
+    XImage im[kMaxBatch];
+    int count;
+};
+hipError_t launch_x_image(const XImageBatch& b, hipStream_t stream);
 struct GwLinear {
     const uint32_t* qweight;
     const uint32_t* qzeros;
@@ -135,7 +140,13 @@ struct FewBatch {
     int count, M, mb, wg_total;
 };
 uint64_t x_rows_bytes(int M, int K);
-hipError_t launch_x_rows(const void* x, bool f32, void* img, int M, int K, hipStream_t stream);
+// the images of up to kMaxBatch inputs of M rows in one launch
+struct XRows {
+    const void* x[kMaxBatch];  // [M, K] fp32 or fp16
+    uint32_t __attribute__((ext_vector_type(4)))* img[kMaxBatch];
+    int K[kMaxBatch], count, M;
+};
+hipError_t launch_x_rows(const XRows& a, bool f32, hipStream_t stream);
 hipError_t launch_gemm_few(FewBatch& b, hipStream_t stream);
 
 // Prefill GEMM over many linears in one persistent launch (M > 16, fp16 x, groups a multiple of
