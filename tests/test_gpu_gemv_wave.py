@@ -173,9 +173,9 @@ def test_image_past_the_workspace(ctx):
     w.release()
 
 
-@pytest.mark.parametrize("M,K", [(3, 8448), (3, 8576), (9, 16128), (9, 16256)])
-def test_both_sides_of_the_longest_k(ctx, M, K):
-    run(ctx, M, [(K, 68)], ql.DTYPE_F32, False, True, "any")
+@pytest.mark.parametrize("M,K,N", [(3, 8448, 2052), (3, 8576, 2052), (9, 5760, 5124), (9, 12160, 5124)])
+def test_both_sides_of_the_longest_k(ctx, M, K, N):
+    run(ctx, M, [(K, N)], ql.DTYPE_F32, False, True, "any")
 
 
 @pytest.mark.parametrize("M", [5, 16])

@@ -2091,10 +2091,11 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
     // rows 12.5 -> 8.2; 8.3; above a thousand the dequantization repeated per 32 rows tells: 256 rows of 896 -> 18944
     // 19.0 -> 26.3). A wave's part of K is a serial chain, so a longer K needs more of them: from 160 on (77 rows of
     // 3584 x 3584 17.3 -> 12.7; 17.7 -> 14.5, 64 of 3584 -> 5120 20.0 -> 12.3; 20.5 -> 14.1, 33 of 5504 -> 6144 17.3 ->
-    // 15.4; 18.7 -> 18.8, but 64 of 4864 -> 896 10.6 -> 14.6), and past 6144, where from HBM the chain takes about 2.2 us
-    // per 1024, 208 (128 rows of 18944 -> 3584 47.4 -> 40.5; 48.1 -> 47.9, but 77 45.2 -> 39.3; 45.5 -> 47.1), or 384 with
-    // two row tiles, which the other forms' 64 rows fit (33 of 18944 -> 13824 81 -> 57; 83 -> 75, but -> 10240
-    // 61 -> 57; 63 -> 73).
+    // 15.4; 18.7 -> 18.8, 77 of 18944 -> 3584 45.2 -> 39.3; 45.7 -> 46.8, but 64 of 4864 -> 896 10.6 -> 14.6). Two row
+    // tiles, which the other forms' 64 rows fit, need to fill a workgroup or two a CU to three quarters past 8192, where
+    // from HBM the chain takes about 2.2 us per 1024 (46 of 13184 -> 2 x 3624, 228 tiles, 35.5 -> 28.8; 40.6 -> 35.5, 33 of
+    // 18944 -> 13824, 432, 81 -> 57; 83 -> 75, but -> 10240, 320, 61 -> 57; 63 -> 73, 64 -> 5120, 160, 39 -> 39; 42 -> 47, 37 of
+    // 14080 -> 3 x 5632, 528, 61 -> 63; 65 -> 80).
     long wgs = 0, n = 0;
     int max_k = 0;
     for (int i = 0; i < count; i++) {
@@ -2103,8 +2104,9 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
         n += descs[i].N;
         max_k = std::max(max_k, descs[i].K);
     }
-    const long least = max_k <= 6144 || M <= 32 ? 160 : M <= 64 ? 384 : 208;
-    if (wgs > (max_k <= 2048 ? 1024 : 1200) || (max_k > 2048 && (wgs < least || n < 2048))) return false;
+    if (wgs > (max_k <= 2048 ? 1024 : 1200) || (max_k > 2048 && (wgs < 160 || n < 2048))) return false;
+    const long rounds = (wgs + ctx->cu_count - 1) / ctx->cu_count;
+    if (max_k > 8192 && M > 32 && M <= 64 && (rounds > 2 || 4 * wgs < 3 * rounds * ctx->cu_count)) return false;
     uint64_t off[ql::kMaxBatch], bytes = 0;
     int first[ql::kMaxBatch];                               // the linear whose image linear i reads
     for (int i = 0; i < count; i++) {
@@ -2158,28 +2160,34 @@ bool few_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql_arena
 
 namespace {
 
-// The longest K at which the products over images are the faster form for n columns in all, with weights that a cache
-// holds and with weights from HBM (as decode's are). A wave's part of K is a chain of groups whose loads
-// wait for each other, 1.1 us per 1024 of K where every CU has a workgroup at most (n <= 16 CUs), 2.1 to 3.4 above;
-// gemv_mfma_kernel's time grows with the rows instead. Measured (us, gemv_mfma_kernel -> this, cached; HBM), per band
-// of n on either side of its line:
-//   n <= 16 CUs: M = 3 8192 -> 4096 12.5 -> 9.1; 14.0 -> 13.2, 9472 -> 4096 12.5 -> 9.7; 14.2 -> 15.1; M = 5 11008 -> 4096
-//     17.2 -> 10.6; 18.6 -> 16.2, 18944 -> 4096 21.7 -> 16.5; 22.3 -> 24.3; M = 8 3584 -> 3584 16.6 -> 7.2; 17.5 -> 9.0,
-//     18944 -> 3584 28.8 -> 17.5; 30.4 -> 25.0; M = 9 (two fragments) 11008 -> 4096 24.0 -> 16.7; 25.6 -> 22.2, 18944 -> 4096
-//     31.6 -> 26.1; 32.2 -> 34.3
-//   to 20 CUs: M = 5 3584 -> 5120 14.0 -> 8.3; 15.6 -> 11.3, 6400 -> 5120 15.1 -> 10.7; 16.5 -> 17.1
-//   to 32 CUs: M = 4 3072 -> 8000 10.2 -> 8.1; 11.5 -> 10.8, 3584 -> 8000 10.1 -> 8.8; 11.4 -> 11.8; M = 8 6400 -> 8000
-//     17.7 -> 12.4; 19.2 -> 17.4, 11008 -> 8000 23.2 -> 18.2; 24.0 -> 25.4
-//   above: M = 5 2048 -> 10240 11.1 -> 8.0; 12.9 -> 10.9, 3584 -> 2 x 18944 22.5 -> 19.8; 25.1 -> 26.1; M = 8 3584 -> 2 x 18944
-//     26.2 -> 19.9; 29.2 -> 26.2, 11008 -> 10240 26.4 -> 24.3; 28.1 -> 33.4; M = 9 3584 -> 2 x 18944 37.1 -> 25.6;
-//     38.3 -> 34.2, 5760 -> 18816 29.2 -> 23.9; 30.6 -> 31.9
-// From 14 rows on it is faster throughout (M = 16 18944 -> 10240 83 -> 46; 85 -> 62).
-int gemv_wave_max_k(int M, long n, int cu_count)
+// The longest K at which `count` products over images, of n columns in all, are the faster form. A wave's part of K is
+// a chain of groups whose loads wait for each other, 1.1 us per 1024 of K with weights from HBM where every CU has a
+// workgroup at most (16 columns a CU), 2.1 to 3.4 above; gemv_mfma_kernel's time grows with the rows instead, and
+// with the linears, each of which it splits by itself. The lines lie where the two forms' times, cached weights
+// and weights from HBM taken together, are equal over 405 random shapes of 3 to 16 rows. Measured (us,
+// gemv_mfma_kernel -> this, cached; HBM), on either side:
+//   up to 4 columns a CU: M = 3 18944 -> 512 22.8 -> 15.3; 23.3 -> 24.0; up to 8: M = 3 9472 -> 2048 14.3 -> 9.7; 15.6 ->
+//     14.5, 14848 -> 2048 15.0 -> 12.2; 16.5 -> 19.5; M = 9 (two fragments) 18944 -> 2048 32.8 -> 24.7; 34.2 -> 34.3
+//   up to 16: M = 3 8192 -> 4096 12.5 -> 9.1; 14.0 -> 13.2, 11008 -> 4096 12.8 -> 10.5; 14.5 -> 16.1; M = 4 11008 -> 4096
+//     14.8 -> 10.5; 16.4 -> 16.1, 18944 -> 3584 19.2 -> 17.1; 21.3 -> 24.5; M = 5 18944 -> 3584 22.5 -> 17.1; 24.5 -> 24.6;
+//     M = 8 3584 -> 3584 16.6 -> 7.2; 17.5 -> 9.0, 18944 -> 3584 28.8 -> 17.5; 30.4 -> 25.0
+//   up to 20: M = 5 6400 -> 5120 15.1 -> 10.7; 16.5 -> 17.1, 11008 -> 5120 17.8 -> 17.9; 20.2 -> 26.6
+//   up to 32: M = 4 3584 -> 8000 10.1 -> 8.8; 11.4 -> 11.8, 6400 -> 8000 12.1 -> 12.4; 14.5 -> 17.3; M = 8 6400 -> 8000
+//     17.7 -> 12.4; 19.2 -> 17.4, 18944 -> 8000 31.3 -> 27.6; 33.3 -> 39.7
+//   more: M = 5 3584 -> 18944 16.7 -> 14.1; 18.9 -> 19.0, 6400 -> 10240 17.7 -> 17.5; 19.9 -> 23.1; M = 8 6400 -> 10240 21.3 ->
+//     17.5; 23.5 -> 23.4, 11008 -> 10240 26.4 -> 24.3; 28.1 -> 33.4; M = 11 10240 -> 18944 1.37 and 1.01 times faster
+//   several linears: M = 5 4096 -> 3 x 3576 17.1 -> 12.2; 18.8 -> 16.6, 16768 -> 3 x 5048 1.24 times faster; 0.91
+int gemv_wave_max_k(int M, int count, long n, int cu_count)
 {
-    if (M >= 14) return INT32_MAX;
-    if (n <= 16L * cu_count) return (M <= 8 ? 2816 : 1792) * M;
-    if (n <= 20L * cu_count) return (M <= 8 ? 1200 : 768) * M;
-    return (n < 32L * cu_count ? 832 : M <= 8 ? 640 : 512) * M;
+    const long per = (n + cu_count - 1) / cu_count;        // columns a CU
+    if (M >= 13 || per <= 4 || (per <= 8 && M > 8)) return INT32_MAX;
+    const int k = per <= 8    ? 3840
+                  : per <= 16 ? (M <= 4 ? 2816 : M <= 8 ? 3840 : 2112)
+                  : per <= 20 ? (M <= 8 ? 1920 : 1344)
+                  : M >= 10   ? 1536
+                  : per < 32  ? 1344
+                              : (M <= 8 ? 1080 : 960);
+    return k * M * (count > 1 ? 2 : 1);
 }
 
 // Decode linears (M <= 16, checked and aligned) over images of x in a workspace: a launch for the
@@ -2188,7 +2196,7 @@ bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql
                      const uint64_t* x_offs, int x_dtype, int M, const uint64_t* y_offs, void* fixed, int* rc)
 {
     // At M = 1, 2 the image's launch costs more than it saves, at M = 3, 4 where there are many columns or K is short
-    // (M = 4: 3584 -> 2 x 18944 20.1 -> 20.7 us).
+    // (M = 4: 3584 -> 2 x 18944 20.1 -> 20.7 us, M = 3: 2048 -> 64 6.8 -> 7.1).
     long n = 0;
     int min_k = INT32_MAX, max_k = 0;
     for (int i = 0; i < count; i++) {
@@ -2196,7 +2204,7 @@ bool gemv_wave_batch(ql_ctx* ctx, int count, const ql_gptq_desc* descs, const ql
         min_k = std::min(min_k, descs[i].K);
         max_k = std::max(max_k, descs[i].K);
     }
-    if (M < 3 || (M < 5 && (n >= 32L * ctx->cu_count || min_k < 2048)) || max_k > gemv_wave_max_k(M, n, ctx->cu_count)) return false;
+    if (M < 3 || (M < 5 && (n >= 32L * ctx->cu_count || min_k < (M == 3 ? 2304 : 2048))) || max_k > gemv_wave_max_k(M, count, n, ctx->cu_count)) return false;
     uint64_t off[ql::kMaxBatch], bytes = 0;
     int first[ql::kMaxBatch];                               // the linear whose image linear i reads
     for (int i = 0; i < count; i++) {
